@@ -20,7 +20,8 @@
 //                      logit; without one (kLogits false: one pass) it writes
 //                      no logits, only that word and the tile's second word (a
 //                      bound on its other logits and the maximum's index).
-//   lm_gemm_narrow_kernel  the same for up to 64 rows, one wave per tile,
+//   lm_gemm_narrow_kernel  the same for up to 64 rows, one wave per tile and 32
+//                      rows on v_mfma_i32_32x32x32_i8,
 //                      logits always written (to the workspace if the caller
 //                      keeps none) with both words; with up to
 //                      kFusedQuantRows rows each workgroup quantises the
@@ -56,6 +57,8 @@ namespace pb {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
@@ -71,8 +74,9 @@ constexpr uint32_t kGemmThreads = 256;  // four waves
 // the nibble unpacking is shared by a wave's rows; 64 rows need 213 VGPRs).
 constexpr uint32_t kRowsPerGroup = 128;
 // Batches up to kNarrowRows take lm_gemm_narrow_kernel (measured per step,
-// Q4_0 / Q8_0: B = 64 74.8 / 73.7 us against 92.0 / 98.1 with the wide kernel;
-// B = 128 119.2 / 121.9 against 103.6 / 108.6).
+// Q4_0 / Q8_0: B = 64 43.2 / 54.6 us against 57 / 69 for 65 rows with the wide
+// kernel; B = 100 68.5 / 85.6 with four row groups of the narrow form, against
+// 64.1 / 81.5 wide).
 constexpr uint32_t kWordsPerRow = kVocab / 32;
 // Blocks of 32 in Qwen2.5-0.5B's hidden state of 896: the width whose block
 // loops are unrolled whole.
@@ -376,14 +380,14 @@ __device__ __forceinline__ uint32_t tile_second_word(const uint32_t (&ow)[4], ui
   return (((other >> 6) + 1u) << 6) | (first & kSecondIndexMask);
 }
 
-// ---- a wave's results for one 64-id tile ----
+// ---- a wide wave's results for one 64-id tile, logits kept ----
 // total[rt][c][i] is row base_row + lane_row + 16 rt + i, id 64 tile + 4n + c,
 // where base_row is the first row of the wave's group of group_rows rows and
 // lane_row the lane's row of step 0 inside it (lanes 16q .. 16q+15 hold rows
 // 4q + i of each row tile, four consecutive ids per lane).  For the real rows among
 // result registers i < kI: stores the raw logits and the order word of the
 // tile's largest raw logit (kNonFiniteTile when one of them is infinite or
-// NaN), and with kSecond the tile's second word.  The repetition penalty is
+// NaN).  The repetition penalty is
 // not applied here: the selection applies it to the few tiles it reads (it
 // never raises a value, so the raw maximum bounds the penalised ones).
 // The logits go out as buffer stores over the group's real rows: a padding
@@ -395,8 +399,8 @@ __device__ __forceinline__ uint32_t tile_second_word(const uint32_t (&ow)[4], ui
 // Measured per 256-row step: Q8_0 161.3-162.0 -> 142.1-149.8 us, Q4_0 about
 // even (128.9-130.0 -> 129.4-134.9 us, HIP events 129.0-131.5 ->
 // 129.4-130.4 us).
-template <int kRT, int kI, bool kSecond>
-__device__ __forceinline__ void write_tile(const LmParams& p, const float (&total)[kRT][4][4],
+template <int kRT, int kI>
+__device__ __forceinline__ void write_tile_logits(const LmParams& p, const float (&total)[kRT][4][4],
                                            uint32_t base_row, uint32_t group_rows,
                                            uint32_t lane_row, uint32_t tile, uint32_t n) {
   constexpr int kSteps = kRT * kI;
@@ -409,7 +413,6 @@ __device__ __forceinline__ void write_tile(const LmParams& p, const float (&tota
       p.logits + (size_t)base_row * ld, (short)0, (int)(real * ld * 4u), kBufferFlags);
   const uint32_t lane_off = (lane_row * ld + v0 + 4u * n) * 4u;
   uint32_t o[kSteps];
-  uint32_t ow[kSteps][4];
 #pragma unroll
   for (int s = 0; s < kSteps; ++s) {
     const int rt = s / kI, i = s % kI;
@@ -418,42 +421,20 @@ __device__ __forceinline__ void write_tile(const LmParams& p, const float (&tota
                                            logits, lane_off + (uint32_t)(16 * rt + i) * ld * 4u, 0,
                                            kNonTemporal);
     o[s] = lane_tile_word(y);
-    if constexpr (kSecond) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) ow[s][c] = order_word(y[c]);
-    }
   }
 #pragma unroll
   for (int s = 0; s < kSteps; ++s) o[s] = row16_max_u32(o[s]);
-  uint32_t sec[kSteps];
-  if constexpr (kSecond) {
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) sec[s] = tile_second_word(ow[s], o[s], n);
-  }
   if (n != 0u) return;
-  if constexpr (kSecond) {
-    // the narrow GEMM: plain stores of the real rows' words (its one-row
-    // step measured 0.3 us slower with the buffer stores below)
+  // the tile words through a resource over the same real rows: a store of
+  // a padding row falls outside it and is dropped (no row test, 32-bit
+  // offsets: 21 fewer VALU instructions per wave of the wide GEMM)
+  const __amdgpu_buffer_rsrc_t tm = __builtin_amdgcn_make_buffer_rsrc(
+      p.tilemax + (size_t)base_row * kTilesPerRow, (short)0, (int)(real * kTilesPerRow * 4u),
+      kBufferFlags);
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-      const uint32_t row = base_row + lane_row + 16u * (uint32_t)(s / kI) + (uint32_t)(s % kI);
-      if (row < p.rows) {
-        p.tilemax[(size_t)row * kTilesPerRow + tile] = o[s];
-        p.tilesec[(size_t)row * kTilesPerRow + tile] = sec[s];
-      }
-    }
-  } else {
-    // the tile words through a resource over the same real rows: a store of
-    // a padding row falls outside it and is dropped (no row test, 32-bit
-    // offsets: 21 fewer VALU instructions per wave of the wide GEMM)
-    const __amdgpu_buffer_rsrc_t tm = __builtin_amdgcn_make_buffer_rsrc(
-        p.tilemax + (size_t)base_row * kTilesPerRow, (short)0, (int)(real * kTilesPerRow * 4u),
-        kBufferFlags);
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-      const uint32_t row = lane_row + 16u * (uint32_t)(s / kI) + (uint32_t)(s % kI);
-      __builtin_amdgcn_raw_buffer_store_b32(o[s], tm, (row * kTilesPerRow + tile) * 4u, 0, 0);
-    }
+  for (int s = 0; s < kSteps; ++s) {
+    const uint32_t row = lane_row + 16u * (uint32_t)(s / kI) + (uint32_t)(s % kI);
+    __builtin_amdgcn_raw_buffer_store_b32(o[s], tm, (row * kTilesPerRow + tile) * 4u, 0, 0);
   }
 }
 
@@ -833,274 +814,490 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
   }
 
   if constexpr (kLogits)
-    write_tile<2, 4, false>(p, total, group0, kRowsPerGroup, lrow0 + 4u * q, tile, n);
+    write_tile_logits<2, 4>(p, total, group0, kRowsPerGroup, lrow0 + 4u * q, tile, n);
   else
     write_tile_words<2, 4>(p, total, group0, kRowsPerGroup, lrow0 + 4u * q, tile, n);
 }
 
-// ---- the head for narrow batches (up to 64 rows) ----
-// The wide kernel stages the scales of 128 rows in LDS and gives each wave
-// 32 rows of one 64-id tile; with few rows most of that work is padding.
-// Here one wave takes one 64-id tile and 16 kRT rows (one MFMA row tile up
-// to 32 rows, two above), four waves per workgroup (two for the Q8_0 head
-// up to 32 rows) over consecutive tiles, the grid's y over the row groups.
-// Each block's weight and activation
-// scales are loaded with its operands (four fp16 weight scales and 4 kRT
-// activation scales per lane), and the loads run kSets - 1 blocks ahead in
-// rotating operand sets: with one wave per tile, the memory in flight per
-// wave is what keeps the weights streaming.  The epilogue is the wide
-// kernel's, for both formats; a Q4_0 tile flagged at pack time for an
-// infinite or NaN weight scale takes the subtract-then-multiply form for all
-// its blocks.  The loop body has no branch: at a branch's join the compiler
-// waits for every load in flight, which would undo the loads issued ahead.
-// For the same reason the Q4_0 block loop is unrolled whole at the model's
-// width (kNB = 28): in the loop form the compiler copies the next block's
-// operands between registers at the loop edge and waits for every load
-// there.  With at most four rows every real row is result register i < kI of lanes
-// 0 .. 15, so the epilogue of the other registers (padding rows) is left
-// out: kI = 1 for one conversation.
+// ---- a narrow wave's results for one 64-id tile ----
+// total[ct][i] of lane l = 32 h + j is row base_row + wave_row + 8 (i / 4) + 4 h + i % 4,
+// id 64 tile + 2 j + ct, for i < kRegs (the MFMA's result layout).
+// base_row is the first row of the workgroup's group of group_rows rows and
+// wave_row the wave's first row in it.
 //
-// kFused (at most kFusedQuantRows rows): each workgroup quantises the rows'
-// activations itself, into LDS, instead of reading them from lm_quant_kernel
-// -- one launch less per step.  The first blocks' weights are requested
-// before the quantisation, so it overlaps their latency.
+// Stored for the real rows: the raw logits, and per (row, tile)
+// the order word of the largest raw logit (kNonFiniteTile when one of them is
+// infinite or NaN) and the second word (kSecondIndexMask).  The repetition
+// penalty is not applied here: the selection applies it to the few tiles it
+// reads (it never raises a value, so the raw maximum bounds the penalised
+// ones).
+//
+// Every store goes through a resource over the group's real rows: a padding
+// row's store falls outside it and is dropped, so no store needs a row test,
+// and each address is the lane's 32-bit offset plus the step's.  The logits
+// are non-temporal: the selection reads a few tiles of them, and ordinary
+// stores of a 256-row step (155.6 MB) evict the packed weights that a
+// workgroup's waves share through the L2 (Q8_0 step of 256 rows: 161.3-162.0
+// -> 142.1-149.8 us).
+//
+// The words go through LDS (buf: the wave's own 16 rows of kTailStride
+// words), sixteen rows at a time, so that four lanes hold a row, sixteen ids
+// each: the largest of each four ids, the two largest of those four maxima,
+// then the largest one's group read again for its place and second value, and
+// a reduction over four lanes instead of 32.  About 100 vector instructions
+// for 32 rows, against 390 with the same reductions over 16 lanes in
+// registers.  A tie at the maximum, in
+// a group or across, makes the bound on the other logits reach the tile
+// word.  The sign of a zero maximum is not kept: the selection reads a tile
+// whose word is the order word of zero.
+constexpr uint32_t kTailStride = 68;
+constexpr uint32_t kTailWords = 16 * kTailStride;
+template <int kRegs>
+__device__ __forceinline__ void write_tile(const LmParams& p, const v4f (&total)[2][(kRegs + 3) / 4],
+                                           uint32_t base_row, uint32_t group_rows,
+                                           uint32_t wave_row, uint32_t tile, uint32_t lane,
+                                           float* buf) {
+  const uint32_t j = lane & 31u;
+  const uint32_t h = lane >> 5;
+  const uint32_t real = p.rows > base_row ? min(p.rows - base_row, group_rows) : 0u;
+  // the LM heads' logits are [rows][PB_VOCAB]: a group's rows span at most
+  // 64 x 151,936 words
+  const uint32_t ld = (uint32_t)p.logits_ld;
+  const __amdgpu_buffer_rsrc_t logits = __builtin_amdgcn_make_buffer_rsrc(
+      p.logits + (size_t)base_row * ld, (short)0, (int)(real * ld * 4u), kBufferFlags);
+  const uint32_t off0 = ((wave_row + 4u * h) * ld + tile * kTileIds + 2u * j) * 4u;
+#pragma unroll
+  for (int i = 0; i < kRegs; ++i)
+    __builtin_amdgcn_raw_buffer_store_b64(
+        v2u{b_of(total[0][i / 4][i % 4]), b_of(total[1][i / 4][i % 4])}, logits, off0,
+        (8u * ((uint32_t)i >> 2) + ((uint32_t)i & 3u)) * ld * 4u, kNonTemporal);
+  const __amdgpu_buffer_rsrc_t tm = __builtin_amdgcn_make_buffer_rsrc(
+      p.tilemax + (size_t)base_row * kTilesPerRow, (short)0, (int)(real * kTilesPerRow * 4u),
+      kBufferFlags);
+  const __amdgpu_buffer_rsrc_t ts = __builtin_amdgcn_make_buffer_rsrc(
+      p.tilesec + (size_t)base_row * kTilesPerRow, (short)0, (int)(real * kTilesPerRow * 4u),
+      kBufferFlags);
+  if constexpr (kRegs <= 2) {
+    // One or two rows, in the registers of lanes 0 .. 31: reduced there, with
+    // no round trips through LDS at the end of a step that is all latency
+    // (Q4_0, one row: 20.7 -> 20.5 us).
+#pragma unroll
+    for (int i = 0; i < kRegs; ++i) {
+      const float y0 = total[0][0][i], y1 = total[1][0][i];
+      const float probe = __builtin_fmaf(y0, 0.0f, y1 * 0.0f);
+      float m, lo;
+      __asm__("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(y0), "v"(y1));
+      __asm__("v_min_f32 %0, %1, %2" : "=v"(lo) : "v"(y0), "v"(y1));
+      const uint32_t at = 2u * j + (y0 == m ? 0u : 1u);
+      const uint32_t o = probe != probe ? kNonFiniteTile : order_word(m);
+      uint32_t word = row16_max_u32(o);
+      word = max(word, lane_xor(word, 16, lane));
+      uint32_t idx = row16_min_u32(o == word ? at : 0xffu);
+      idx = min(idx, lane_xor(idx, 16, lane));
+      uint32_t other = row16_max_u32(at == idx ? order_word(lo) : o);
+      other = max(other, lane_xor(other, 16, lane));
+      if (lane == 0u) {
+        const uint32_t off = ((wave_row + (uint32_t)i) * kTilesPerRow + tile) * 4u;
+        __builtin_amdgcn_raw_buffer_store_b32(word, tm, off, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(((other & ~kSecondIndexMask) + 64u) | idx, ts, off, 0, 0);
+      }
+    }
+    return;
+  }
+  const uint32_t qd = lane & 3u;  // quarter of the row
+  const float* mine = buf + (lane >> 2) * kTailStride + 16u * qd;
+  auto pass = [&](auto half_tag) __attribute__((always_inline)) {
+    constexpr int half = decltype(half_tag)::value;
+    // the rows past kRegs are left as they are: their words are not stored
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const int i = 8 * half + r;
+      if (i < kRegs)
+        *reinterpret_cast<v2f*>(buf + (8u * ((uint32_t)r >> 2) + 4u * h + ((uint32_t)r & 3u)) * kTailStride +
+                                2u * j) = v2f{total[0][i / 4][i % 4], total[1][i / 4][i % 4]};
+    }
+    __builtin_amdgcn_wave_barrier();
+    v4f v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const v4f*>(mine + 4 * k);
+    float probe = 0.0f;
+    float gm[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) probe = __builtin_fmaf(v[k][c], 0.0f, probe);
+      // (only used when every value is finite: no quietening of NaN operands)
+      __asm__("v_max3_f32 %0, %1, %2, %3\n\tv_max_f32 %0, %0, %4"
+              : "=&v"(gm[k])
+              : "v"(v[k].x), "v"(v[k].y), "v"(v[k].z), "v"(v[k].w));
+    }
+    float m3, md, lo, m, sg;
+    __asm__("v_max3_f32 %0, %1, %2, %3" : "=v"(m3) : "v"(gm[0]), "v"(gm[1]), "v"(gm[2]));
+    __asm__("v_med3_f32 %0, %1, %2, %3" : "=v"(md) : "v"(gm[0]), "v"(gm[1]), "v"(gm[2]));
+    __asm__("v_min_f32 %0, %1, %2" : "=v"(lo) : "v"(m3), "v"(gm[3]));
+    __asm__("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(m3), "v"(gm[3]));
+    __asm__("v_max_f32 %0, %1, %2" : "=v"(sg) : "v"(md), "v"(lo));
+    uint32_t k = gm[2] == m ? 8u : 12u;
+    k = gm[1] == m ? 4u : k;
+    k = gm[0] == m ? 0u : k;
+    const v4f w = *reinterpret_cast<const v4f*>(mine + k);
+    float s2;
+    __asm__("v_max3_f32 %0, %1, %2, %3" : "=v"(m3) : "v"(w.x), "v"(w.y), "v"(w.z));
+    __asm__("v_med3_f32 %0, %1, %2, %3" : "=v"(md) : "v"(w.x), "v"(w.y), "v"(w.z));
+    __asm__("v_min_f32 %0, %1, %2" : "=v"(lo) : "v"(m3), "v"(w.w));
+    __asm__("v_max3_f32 %0, %1, %2, %3" : "=v"(s2) : "v"(md), "v"(lo), "v"(sg));
+    uint32_t c = w.z == m ? 2u : 3u;
+    c = w.y == m ? 1u : c;
+    c = w.x == m ? 0u : c;
+    const uint32_t at = 16u * qd + k + c;
+    const uint32_t o = probe != probe ? kNonFiniteTile : order_word(m);
+    // over the row's four lanes
+    uint32_t word = max(o, dpp_or_zero<0xB1>(o));
+    word = max(word, dpp_or_zero<0x4E>(word));
+    uint32_t idx = o == word ? at : 0xffu;
+    idx = min(idx, dpp_or_zero<0xB1>(idx));
+    idx = min(idx, dpp_or_zero<0x4E>(idx));
+    uint32_t other = at == idx ? order_word(s2) : o;
+    other = max(other, dpp_or_zero<0xB1>(other));
+    other = max(other, dpp_or_zero<0x4E>(other));
+    if (qd == 0u) {
+      const uint32_t off = ((wave_row + 16u * (uint32_t)half + (lane >> 2)) * kTilesPerRow + tile) * 4u;
+      __builtin_amdgcn_raw_buffer_store_b32(word, tm, off, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b32(((other & ~kSecondIndexMask) + 64u) | idx, ts, off, 0, 0);
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  pass(std::integral_constant<int, 0>{});
+  if constexpr (kRegs > 8) pass(std::integral_constant<int, 1>{});
+}
+
+// ---- the head for narrow batches (up to 64 rows) ----
+// The wide kernel stages the scales of 128 rows in LDS and gives the four
+// waves of a workgroup one 64-id tile; with few rows most of that work is
+// padding.  Here a wave takes one tile and one group of 32 rows (kGroups row
+// groups per workgroup, so that a tile's weights are read by the waves of one
+// workgroup), and of its 16 result registers per column tile only the kRegs
+// that hold real rows go through the epilogue: registers 0 .. 3 of both lane
+// halves hold rows 0 .. 7, 0 .. 7 rows 0 .. 15, and so on.
+//
+// One v_mfma_i32_32x32x32_i8 multiplies 32 rows by 32 ids over one whole
+// 32-element block.  Lane l = 32 h + j holds row (A) / column (B) j and 16
+// contraction slots as four registers: slots 16 h .. 16 h + 15, which carry
+// block elements 4 q .. 4 q + 3 and 16 + 4 q .. 16 + 4 q + 3 for q = 2 h, then
+// for q = 2 h + 1 -- one packed Q4_0 weight word gives both halves of a q, its
+// low nibbles and its high nibbles.  Result register i of the lane is
+// D[8 (i / 4) + 4 h + i % 4][j].  Column j of column tile ct is id
+// 64 tile + 2 j + ct, so that the lane's two ids are neighbours in memory.
+//
+// The accumulator starts at the bit pattern of M = 1.5 * 2^23 for both
+// formats, so each result word read as binary32 is exactly M + dot.  The Q4_0
+// epilogue is the wide kernel's; for Q8_0, x - M is f32(dot) exactly (a
+// subtraction issues at twice the rate of a conversion, below), then
+// add(total, mul(f32(dot), mul(ws, a_scale))).  A Q4_0 tile flagged at pack
+// time for an infinite or NaN weight scale is computed again with the
+// subtract-then-multiply form.
+//
+// What bounds it: up to about 16 rows the read of the head; above, the issue
+// of vector instructions.  Measured on MI355X with four waves on a SIMD
+// (cycles of the SIMD per wave instruction): fma, mul, add, sub, and, or and
+// mov of vector registers 2.2-2.4 -- two waves issue together -- but 4.1-4.2
+// with a scalar register operand, and for conversions, shifts, max, max3,
+// compares and anything with DPP; and while an MFMA runs, vector instructions
+// issue one at a time.  A tile of 32 rows by 64 ids and one block is 96 fma,
+// mul and add: 108 ns alone, 127-129 ns beside two 32x32x32 MFMAs (32 cycles
+// each) and 140 ns beside the eight 16x16x32 ones (16 cycles each) that give
+// the same products.  So: the large MFMA, and masks and scales in vector
+// registers.  The block loop is software-pipelined in two phases: while column
+// tile 0 of block b goes through the epilogue the MFMA of its column tile 1
+// runs, and beside that one's epilogue the MFMA of the next block's column
+// tile 0; each quad of activation scales is reloaded from LDS for the next
+// block as soon as its last use is out.  The packed operands are requested two
+// blocks ahead; one block ahead for the Q8_0 head with one row group, which
+// has twice the bytes per block (one row 33.0 -> 31.4 us, 16 rows 38.6 -> 37.5;
+// the Q4_0 head one block ahead: one row 20.7 -> 22.1).  (The same loop with
+// four row groups and LDS-staged weight scales was no faster than the wide
+// kernel: 256 rows 116-125 us a step against 115-122.)
 constexpr uint32_t kMaxBlocks = 2048 / 32;
-template <bool kQ8, int kRT, int kSets, int kI, bool kFused, int kNB, int kNW>
-__global__ __launch_bounds__(64 * kNW) void lm_gemm_narrow_kernel(LmParams p) {
-  static_assert(kI == 4 || kRT == 1, "partial rows only with one row tile");
-  static_assert(!kFused || (kRT == 1 && kI <= (int)kFusedQuantRows), "fused rows fit one row tile");
-  // kFused: [block][row] quants (8 words) and scales / 16 of the real rows
-  __shared__ __align__(16) uint32_t aq_lds[kFused ? kMaxBlocks : 1][kFused ? kFusedQuantRows : 1][8];
-  __shared__ __align__(16) float as_lds[kFused ? kMaxBlocks : 1][kFused ? kFusedQuantRows : 1];
-  const uint32_t lane = threadIdx.x & 63u;
-  // the tile is wave-uniform: held in scalar registers, so every load below
-  // is a scalar base plus a 32-bit lane offset, with no 64-bit address
-  // arithmetic per lane
-  const uint32_t tile_raw = blockIdx.x * (uint32_t)kNW + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const bool live_wave = tile_raw < kTilesPerRow;
-  // waves past the last tile work on the last one (and store nothing), so
-  // that every wave reaches the workgroup barrier of the fused quantisation
-  const uint32_t tile = live_wave ? tile_raw : kTilesPerRow - 1u;
-  if (!kFused && !live_wave) return;  // whole wave, no barrier follows
-  const uint32_t n = lane & 15u;
-  const uint32_t q = lane >> 4;
-  const uint32_t row0 = blockIdx.y * (16u * kRT);  // first row of the wave's group
-  // kNB > 0: the width is 32 kNB, known at compile time (the block loop is
-  // unrolled whole, so no loaded register crosses a loop edge)
-  const uint32_t blocks = kNB > 0 ? (uint32_t)kNB : p.cols / 32u;
-  const uint32_t last = blocks - 1u;
-  constexpr uint32_t kWords = kQ8 ? 2u : 1u;  // uint4 of packed weights per lane and block
+template <bool kQ8, int kGroups, int kRegs, bool kFused, int kWaves>
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRegs >= 12 && !(kQ8 && kGroups == 1) ? 3 : 4))) void lm_gemm_narrow_kernel(LmParams p) {
+  constexpr uint32_t kRows = 32u * kGroups;      // rows per workgroup
+  constexpr uint32_t kTiles = kWaves / kGroups;  // tiles per workgroup
+  constexpr uint32_t kThreads = 64u * kWaves;
+  constexpr int kQuads = (kRegs + 3) / 4;        // result quads in use
+  constexpr uint32_t kSets = kQ8 && kGroups == 1 ? 1 : 2;
+  constexpr uint32_t kActSets = kSets;
+  static_assert(!kFused || (kGroups == 1 && kRegs <= 4), "fused rows fit one result quad");
+  // Dynamic LDS: the activation scales (/ 16 for Q4_0) by row group, block and row; kFused: then
+  // each block's quants, a real row's eight words each and a row of zeros.
+  extern __shared__ __align__(16) float lds[];
+  const uint32_t blocks = p.cols / 32u;
+  const uint32_t group_words = blocks * 32u;  // of one row group's scales
+  float* act_scale = lds;
+  const uint32_t tid = threadIdx.x;
+  const uint32_t lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t j = lane & 31u;  // MFMA row (A) / column (B)
+  const uint32_t h = lane >> 5;   // contraction half; result rows 8 g + 4 h + ..
+  // Consecutive tiles run on the same XCD (xcd_contiguous_item): every
+  // (row, tile) gets two 4-byte words in row-major arrays, and the
+  // words of up to eight neighbouring tiles share a 32-byte sector, which
+  // leaves an XCD's L2 whole only when the neighbours were written through
+  // that L2.  With tile = block index the neighbours sat on eight different
+  // XCDs: 8 x the words' bytes written (39.7 MB instead of 4.9 MB per
+  // 256-row one-pass step, WRITE_SIZE).  The row groups of one tile are
+  // consecutive items, so they run on one XCD at about the same time and the
+  // head leaves HBM once (group-major items read it once per group).
+  const uint32_t item = xcd_contiguous_item(blockIdx.x + blockIdx.y * gridDim.x,
+                                            gridDim.x * gridDim.y);
+  const uint32_t tile_raw = item / gridDim.y * kTiles + wave / kGroups;
+  const uint32_t tile = min(tile_raw, kTilesPerRow - 1u);
+  const uint32_t group0 = item % gridDim.y * kRows;
+  const uint32_t wave_row = wave % kGroups * 32u;  // first row inside the workgroup's rows
+  const uint32_t rw0 = group0 + wave_row;
+  const bool live = rw0 < p.rows && tile_raw < kTilesPerRow;  // else the whole wave idles
   constexpr uint32_t kTile = kQ8 ? kTileBytesQ8 : kTileBytes;
-
-  // Each load is a wave-uniform base plus one 32-bit byte offset (the block's
-  // uniform part + the lane's part).  The widths of at most 2048 keep the
-  // packed head under 330 MB, so every offset fits.
-  const uint8_t* a_base = reinterpret_cast<const uint8_t*>(p.act_q);
-  const uint32_t a_stride = p.rows_pad * 32u;  // bytes per block
-  const uint32_t a_off = (row0 + n) * 32u + 8u * q;
-  const uint8_t* w_base = p.weights;
+  // The operands are buffer loads: a lane's byte offset is fixed, the block's
+  // offset is a scalar, so a load costs no VALU address arithmetic (three to
+  // five instructions per block otherwise).  Widths of at most 2048 keep the
+  // packed head under 330 MB, and the activations of at most
+  // PB_LMHEAD_MAX_ROWS rows (the host refuses more) take blocks * rows_pad * 32
+  // <= 512 MB, so every offset and resource size fits in 31 bits.
   const uint32_t w_stride = kTilesPerRow * kTile;  // bytes per block
-  const uint32_t w_off = tile * kTile + 16u * kWords * lane;
-  const uint8_t* ws_base = p.weights;
-  const uint32_t ws_off = blocks * kVocab * (kQ8 ? 32u : 16u) + 2u * tile * kTileIds + 8u * n;
-  const uint8_t* as_base = reinterpret_cast<const uint8_t*>(p.act_s);
-  const uint32_t as_stride = p.rows_pad * 4u;
-  const uint32_t as_off = (row0 + 4u * q) * 4u;
+  const uint32_t w_off = tile * kTile + (kQ8 ? 1024u * h + 16u * j : 512u * h + 8u * j);
+  const uint32_t s_off = tile * (2u * kTileIds) + 4u * j;
+  const uint32_t a_stride = p.rows_pad * 32u;  // bytes per block
+  const uint32_t a_off = (rw0 + j) * 32u + 16u * h;
+  const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(p.weights), (short)0, (int)(blocks * w_stride), kBufferFlags);
+  const __amdgpu_buffer_rsrc_t ws_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint8_t*>(p.weights) + (size_t)blocks * w_stride, (short)0,
+      (int)(blocks * kVocab * 2u), kBufferFlags);
+  const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<int8_t*>(p.act_q), (short)0, kFused ? 0 : (int)(blocks * a_stride), kBufferFlags);
+  float* tail_lds = lds + kGroups * group_words;  // a buffer per wave
+  uint32_t* aq_lds = reinterpret_cast<uint32_t*>(tail_lds + (uint32_t)kWaves * kTailWords);
+  const uint32_t aq_off = min(j, p.rows) * 8u + 4u * h;  // kFused: a padding lane reads the zero row
+  const uint32_t aq_stride = (p.rows + 1u) * 8u;
 
-  // Only the kI activation scales a lane uses are loaded: a register of a
-  // wider load left unused would be taken for a temporary while the load is
-  // in flight, and writing it would wait for every load.
-  typedef float vIf __attribute__((ext_vector_type(kI)));
+  // Packed operands of one block: the lane's 16 activation bytes, and its
+  // weights of both column tiles for q = 2 h and q = 2 h + 1, and the two
+  // ids' fp16 weight scales.
+  typedef typename std::conditional<kQ8, v4u, v2u>::type WeightWords;
   struct Operands {
-    uint64_t a[kRT];
-    v4u raw[kWords];
-    uint64_t ws;    // four fp16 weight scales, ids 4n .. 4n+3
-    vIf as[kRT];    // activation scales / 16 of rows 16 rt + 4q .. 4q + kI - 1
+    WeightWords w[2];
+    uint32_t ws;
   };
-  auto load_w = [&](uint32_t b, Operands& o) {
-    const uint32_t wo = b * w_stride + w_off;
+  auto load_w = [&](uint32_t b, Operands& o) __attribute__((always_inline)) {
+    const uint32_t wb = b * w_stride;
 #pragma unroll
-    for (uint32_t k = 0; k < kWords; ++k)
-      o.raw[k] = *reinterpret_cast<const v4u*>(w_base + (wo + 16u * k));
-    o.ws = *reinterpret_cast<const uint64_t*>(ws_base + (b * (kVocab * 2u) + ws_off));
-  };
-  auto load_a = [&](uint32_t b, Operands& o) {
-    if constexpr (kFused) {
-      // real rows only: lanes n < rows (A) and the q == 0 result registers
-      const uint64_t a = *reinterpret_cast<const uint64_t*>(&aq_lds[b][n & (kFusedQuantRows - 1u)][2u * q]);
-      o.a[0] = n < p.rows ? a : 0ull;
-      vIf v;
-#pragma unroll
-      for (int i = 0; i < kI; ++i) v[i] = q == 0u ? as_lds[b][i] : 0.0f;
-      o.as[0] = v;
-    } else {
-      const uint32_t ao = b * a_stride + a_off;
-#pragma unroll
-      for (int rt = 0; rt < kRT; ++rt)
-        o.a[rt] = *reinterpret_cast<const uint64_t*>(a_base + (ao + 16u * 32u * (uint32_t)rt));
-      const uint32_t so = b * as_stride + as_off;
-#pragma unroll
-      for (int rt = 0; rt < kRT; ++rt)
-        o.as[rt] = *reinterpret_cast<const vIf*>(as_base + (so + 64u * (uint32_t)rt));
+    for (uint32_t k = 0; k < 2; ++k) {
+      if constexpr (kQ8)
+        o.w[k] = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_off + 512u * k, wb, 0);
+      else
+        o.w[k] = __builtin_amdgcn_raw_buffer_load_b64(w_rsrc, w_off + 256u * k, wb, 0);
     }
+    o.ws = __builtin_amdgcn_raw_buffer_load_b32(ws_rsrc, s_off, b * (kVocab * 2u), 0);
   };
-
-  float total[kRT][4][4];
-#pragma unroll
-  for (int rt = 0; rt < kRT; ++rt)
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) total[rt][c][i] = 0.0f;
-  const v4i magic = {(int)kMagicBits, (int)kMagicBits, (int)kMagicBits, (int)kMagicBits};
-  const v4i zero = {0, 0, 0, 0};
-
-  // run() hands each value's term of the block (the reference's rounded
-  // product) to sink(rt, c, i, term); add() adds it to the running total.
-  auto add = [&](int rt, int c, int i, float term) { total[rt][c][i] = total[rt][c][i] + term; };
-  auto run = [&](const Operands& o, auto odd_tag, auto sink) {
-    constexpr bool kOdd = decltype(odd_tag)::value;
-    float wsv[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      wsv[c] = __half2float(__ushort_as_half((unsigned short)(o.ws >> (16 * c))));
-    v4i d[kRT][4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      uint64_t w;
-      if constexpr (kQ8) {
-        const uint32_t raw[8] = {o.raw[0].x, o.raw[0].y, o.raw[0].z, o.raw[0].w,
-                                 o.raw[kWords - 1].x, o.raw[kWords - 1].y, o.raw[kWords - 1].z,
-                                 o.raw[kWords - 1].w};
-        w = (uint64_t)raw[2 * c] | ((uint64_t)raw[2 * c + 1] << 32);
-      } else {
-        const uint32_t raw[4] = {o.raw[0].x, o.raw[0].y, o.raw[0].z, o.raw[0].w};
-        w = (uint64_t)((raw[c] << 4) & 0xf0f0f0f0u) | ((uint64_t)(raw[c] & 0xf0f0f0f0u) << 32);
-      }
-#pragma unroll
-      for (int rt = 0; rt < kRT; ++rt)
-        d[rt][c] = __builtin_amdgcn_mfma_i32_16x16x32_i8((long)o.a[rt], (long)w,
-                                                         kQ8 ? zero : magic, 0, 0, 0);
-    }
-    if constexpr (kQ8) {
-#pragma unroll
-      for (int rt = 0; rt < kRT; ++rt) {
-        float asv[kI];
-#pragma unroll
-        for (int i = 0; i < kI; ++i) asv[i] = o.as[rt][i];
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-          for (int i = 0; i < kI; ++i) {
-            const float scale = wsv[c] * asv[i];
-            sink(rt, c, i, (float)d[rt][c][i] * scale);
-          }
-      }
-    } else {
-      if constexpr (kOdd) {
-#pragma unroll
-        for (int rt = 0; rt < kRT; ++rt) {
-          float asv[kI];
-#pragma unroll
-          for (int i = 0; i < kI; ++i) asv[i] = o.as[rt][i];
-#pragma unroll
-          for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int i = 0; i < kI; ++i) {
-              const float y = (__int_as_float(d[rt][c][i]) - kMagic) * wsv[c];
-              sink(rt, c, i, y * asv[i]);
-            }
-        }
-      } else {
-        float wnv[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) wnv[c] = wsv[c] * -kMagic;
-#pragma unroll
-        for (int rt = 0; rt < kRT; ++rt) {
-          float asv[kI];
-#pragma unroll
-          for (int i = 0; i < kI; ++i) asv[i] = o.as[rt][i];
-#pragma unroll
-          for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int i = 0; i < kI; ++i) {
-              const float y = __builtin_fmaf(__int_as_float(d[rt][c][i]), wsv[c], wnv[c]);
-              sink(rt, c, i, y * asv[i]);
-            }
-        }
-      }
-    }
+  v4i act[kActSets];
+  auto load_a = [&](uint32_t b, v4i& a) __attribute__((always_inline)) {
+    if constexpr (kFused)
+      a = *reinterpret_cast<const v4i*>(&aq_lds[b * aq_stride + aq_off]);
+    else
+      a = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_off, b * a_stride, 0));
   };
-
-  // Block t sits in set t % kSets.  Loads are unconditional (clamped to the
-  // last block).  Whole rounds of kSets blocks run in the loop; the last
-  // blocks (fewer than kSets, already loaded) run after it.  The first
-  // kSets - 1 blocks are requested before anything else (and, with kFused,
-  // before the quantisation and its barrier, which every wave reaches on the
-  // same path).
+  // a Q4_0 tile with an infinite or NaN weight scale (flagged at pack time)
+  const bool odd_tile =
+      !kQ8 && row_word(reinterpret_cast<const uint32_t*>(p.weights + (size_t)blocks * kVocab * 18) + tile) != 0u;
+  // The first blocks' weights are requested before the scales are staged (or
+  // the rows quantised), so their latency overlaps that and its barrier.
   Operands ops[kSets];
+  const uint32_t last = blocks - 1u;
+  if (live) {
 #pragma unroll
-  for (int k = 0; k < kSets - 1; ++k) load_w(min((uint32_t)k, last), ops[k]);
+    for (uint32_t k = 0; k < kSets; ++k) load_w(min(k, last), ops[k]);
+    if constexpr (!kFused) {
+#pragma unroll
+      for (uint32_t k = 0; k < kActSets; ++k) load_a(min(k, last), act[k]);
+    }
+  }
+
   if constexpr (kFused) {
     // the rows' activations, quantised into LDS while those loads fly
-    for (uint32_t pair = threadIdx.x; pair < p.rows * blocks; pair += 64u * kNW) {
+    for (uint32_t pair = tid; pair < p.rows * blocks; pair += kThreads) {
       const uint32_t r = pair / blocks;
       const uint32_t b = pair - r * blocks;
       uint32_t x[32], packed[8];
       float scale16;
       load_block(p, r, b, x);
       quantize_block(x, true, packed, scale16);
-      *reinterpret_cast<v4u*>(&aq_lds[b][r][0]) = v4u{packed[0], packed[1], packed[2], packed[3]};
-      *reinterpret_cast<v4u*>(&aq_lds[b][r][4]) = v4u{packed[4], packed[5], packed[6], packed[7]};
-      as_lds[b][r] = kQ8 ? scale16 * 16.0f : scale16;  // a_scale for the Q8_0 epilogue
+      uint32_t* q = &aq_lds[b * aq_stride + r * 8u];
+      *reinterpret_cast<v4u*>(q) = v4u{packed[0], packed[1], packed[2], packed[3]};
+      *reinterpret_cast<v4u*>(q + 4) = v4u{packed[4], packed[5], packed[6], packed[7]};
+      act_scale[b * 32u + r] = kQ8 ? scale16 * 16.0f : scale16;  // a_scale for the Q8_0 epilogue
     }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int k = 0; k < kSets - 1; ++k) load_a(min((uint32_t)k, last), ops[k]);
-  auto gemm = [&](auto odd_tag) {
-    if constexpr (kNB > 0) {
-#pragma unroll
-      for (int b = 0; b < kNB; ++b) {
-        if (b + kSets - 1 < kNB) {
-          load_w((uint32_t)(b + kSets - 1), ops[(b + kSets - 1) % kSets]);
-          load_a((uint32_t)(b + kSets - 1), ops[(b + kSets - 1) % kSets]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        run(ops[b % kSets], odd_tag, add);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      return;
-    }
-    const uint32_t whole = blocks / kSets * kSets;
-#pragma unroll 1
-    for (uint32_t b = 0; b < whole; b += kSets) {
-#pragma unroll
-      for (int k = 0; k < kSets; ++k) {
-        const uint32_t ahead = min(b + (uint32_t)(k + kSets - 1), last);
-        load_w(ahead, ops[(k + kSets - 1) % kSets]);
-        load_a(ahead, ops[(k + kSets - 1) % kSets]);
-        __builtin_amdgcn_sched_barrier(0);
-        run(ops[k], odd_tag, add);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < kSets - 1; ++k)
-      if (whole + (uint32_t)k < blocks) run(ops[k], odd_tag, add);
-  };
-  if constexpr (kQ8) {
-    gemm(std::false_type{});
+    for (uint32_t b = tid; b < blocks * 2u; b += kThreads)
+      *reinterpret_cast<v4u*>(&aq_lds[(b >> 1) * aq_stride + p.rows * 8u + (b & 1u) * 4u]) =
+          v4u{0u, 0u, 0u, 0u};
   } else {
-    const uint32_t* flags =
-        reinterpret_cast<const uint32_t*>(p.weights + (size_t)blocks * kVocab * 18);
-    if (flags[tile] != 0u) {
-      gemm(std::true_type{});
-    } else {
-      gemm(std::false_type{});
+    // Staged four rows per thread and load (16 bytes; rows_pad is a multiple
+    // of 64, so four rows are all inside the padded batch or all past it), four
+    // loads requested before any is stored.  Rows past the padded batch (only
+    // idle waves use them) read at the end of the resource, which returns
+    // zeros.  lm_quant_kernel stores a_scale / 16 for the Q4_0 epilogue and
+    // a_scale for the Q8_0 one.
+    const uint32_t as_bytes = blocks * p.rows_pad * 4u;
+    const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        p.act_s, (short)0, (int)as_bytes, kBufferFlags);
+    constexpr uint32_t kRowQuads = kRows / 4u;  // four rows per load
+    const uint32_t quads = blocks * kRowQuads;
+    for (uint32_t t0 = tid; t0 < quads; t0 += 4u * kThreads) {
+      v4u as[4];
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t t = t0 + k * kThreads;
+        const uint32_t r = group0 + 4u * (t % kRowQuads);
+        const uint32_t off = r < p.rows_pad ? ((t / kRowQuads) * p.rows_pad + r) * 4u : as_bytes;
+        as[k] = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, off, 0, 0);
+      }
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t t = t0 + k * kThreads;
+        const uint32_t r = 4u * (t % kRowQuads);
+        if (t < quads)
+          *reinterpret_cast<v4u*>(
+              &act_scale[(r >> 5) * group_words + t / kRowQuads * 32u + (r & 31u)]) = as[k];
+      }
     }
   }
-  if (live_wave) write_tile<kRT, kI, true>(p, total, row0, 16u * kRT, 4u * q, tile, n);
+  __syncthreads();
+  if (!live) return;  // whole wave idle (no barrier follows)
+  if constexpr (kFused) {
+#pragma unroll
+    for (uint32_t k = 0; k < kActSets; ++k) load_a(min(k, last), act[k]);
+  }
+
+  v16i magic;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) magic[i] = (int)kMagicBits;
+  __asm__ volatile("" : "+v"(magic));  // held in registers, not made anew in the loop
+  uint32_t mask = 0xf0f0f0f0u;
+  __asm__ volatile("" : "+v"(mask));  // a vector register: see above
+  v4f total[2][kQuads];
+#pragma unroll
+  for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+    for (int g = 0; g < kQuads; ++g) total[ct][g] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  v16i d[2];
+  v4i w;
+  v4f as[kQuads];
+  float ws[2], wn[2];
+
+  const float* as_lds = act_scale + wave % kGroups * group_words + 4u * h;
+  auto load_as = [&](uint32_t b, int g) __attribute__((always_inline)) {
+    as[g] = *reinterpret_cast<const v4f*>(as_lds + b * 32u + 8u * (uint32_t)g);
+  };
+  auto operand = [&](const Operands& o, int ct) __attribute__((always_inline)) -> v4i {
+    if constexpr (kQ8)
+      return v4i{(int)o.w[0][2 * ct], (int)o.w[0][2 * ct + 1], (int)o.w[1][2 * ct],
+                 (int)o.w[1][2 * ct + 1]};
+    else
+      return v4i{(int)((o.w[0][ct] << 4) & mask), (int)(o.w[0][ct] & mask),
+                 (int)((o.w[1][ct] << 4) & mask), (int)(o.w[1][ct] & mask)};
+  };
+  // the block's weight scale of column tile ct, in the epilogue's form
+  auto scale = [&](const Operands& o, int ct) __attribute__((always_inline)) {
+    ws[ct] = __half2float(__ushort_as_half((unsigned short)(o.ws >> (16 * ct))));
+    if constexpr (!kQ8) wn[ct] = ws[ct] * -kMagic;
+  };
+  auto epilogue = [&](int ct, int g) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = 4 * g + r;
+      if (i >= kRegs) continue;
+      const float x = __int_as_float(d[ct][i]);
+      float y;
+      if constexpr (kQ8)
+        y = (x - kMagic) * (ws[ct] * as[g][r]);
+      else
+        y = __builtin_fmaf(x, ws[ct], wn[ct]) * as[g][r];
+      total[ct][g][r] = total[ct][g][r] + y;
+    }
+  };
+  // Block b: its weights in o (column tile 0's operand in w) and activations
+  // in a, the next block's weights in o1; the operands kSets (kActSets) blocks ahead
+  // are requested into o and a.
+  auto block = [&](uint32_t b, Operands& o, Operands& o1, v4i& a, v4i& a1) __attribute__((always_inline)) {
+    const uint32_t ahead = min(b + 1u, last);
+    scale(o, 1);
+    w = operand(o, 1);
+    d[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, w, magic, 0, 0, 0);
+    load_a(min(b + kActSets, last), a);
+    load_w(min(b + kSets, last), o);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < kQuads; ++g) {
+      epilogue(0, g);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    scale(o1, 0);
+    w = operand(o1, 0);
+    d[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a1, w, magic, 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < kQuads; ++g) {
+      epilogue(1, g);
+      load_as(ahead, g);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+#pragma unroll
+  for (int g = 0; g < kQuads; ++g) load_as(0, g);
+  scale(ops[0], 0);
+  d[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(act[0], operand(ops[0], 0), magic, 0, 0, 0);
+  uint32_t b = 0;
+#pragma unroll 1
+  for (; b + kSets <= blocks; b += kSets) {
+#pragma unroll
+    for (uint32_t k = 0; k < kSets; ++k)
+      block(b + k, ops[k], ops[(k + 1) % kSets], act[k % kActSets], act[(k + 1) % kActSets]);
+  }
+#pragma unroll
+  for (uint32_t k = 0; k + 1 < kSets; ++k)
+    if (b + k < blocks)
+      block(b + k, ops[k], ops[(k + 1) % kSets], act[k % kActSets], act[(k + 1) % kActSets]);
+  if constexpr (!kQ8) {
+    // Block by block again with the subtract-then-multiply form.
+    if (odd_tile) {
+#pragma unroll
+      for (int ct = 0; ct < 2; ++ct) {
+#pragma unroll
+        for (int g = 0; g < kQuads; ++g) total[ct][g] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+        for (uint32_t o_b = 0; o_b < blocks; ++o_b) {
+          load_w(o_b, ops[0]);
+          load_a(o_b, act[0]);
+          scale(ops[0], ct);
+          d[ct] = __builtin_amdgcn_mfma_i32_32x32x32_i8(act[0], operand(ops[0], ct), magic, 0, 0, 0);
+#pragma unroll
+          for (int g = 0; g < kQuads; ++g) {
+            load_as(o_b, g);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int i = 4 * g + r;
+              if (i < kRegs)
+                total[ct][g][r] = total[ct][g][r] + ((__int_as_float(d[ct][i]) - kMagic) * ws[ct]) * as[g][r];
+            }
+          }
+        }
+      }
+    }
+  }
+  // the lane number anew: nothing that the tail derives from it is kept through the loop
+  uint32_t none = 0;
+  __asm__ volatile("" : "+s"(none));
+  write_tile<kRegs>(p, total, group0, kRows, wave_row, tile,
+                             __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, none)),
+                             tail_lds + wave * kTailWords);
 }
 
 // A value every lane holds alike, moved to a scalar register so that the
@@ -2081,31 +2278,64 @@ hipError_t launch_lm_pack_q8(const uint8_t* in, uint8_t* out, uint32_t vocab, ui
   return hipGetLastError();
 }
 
-size_t gemm_lds_bytes(uint32_t cols) {
-  return (size_t)(cols / 32u) * (kRowsPerGroup + 2u * kTileIds) * sizeof(float);
+// The wide GEMM; the Q4_0 block loop is unrolled whole at the model's width.
+template <bool kQ8>
+static void launch_gemm_wide(const LmParams& p, hipStream_t stream) {
+  const uint32_t blocks = p.cols / 32u;
+  const dim3 grid(kTilesPerRow, (p.rows + kRowsPerGroup - 1) / kRowsPerGroup);
+  const size_t lds = (size_t)blocks * (kRowsPerGroup + 2u * kTileIds) * sizeof(float);
+  const bool unrolled = !kQ8 && blocks == kModelBlocks;
+  if (p.logits == nullptr) {  // one pass: tile and second words, no logits
+    if (unrolled)
+      hipLaunchKernelGGL((lm_gemm_kernel<kQ8, false, kQ8 ? 0u : kModelBlocks>), grid,
+                         dim3(kGemmThreads), lds, stream, p);
+    else
+      hipLaunchKernelGGL((lm_gemm_kernel<kQ8, false>), grid, dim3(kGemmThreads), lds, stream, p);
+  } else if (unrolled) {
+    hipLaunchKernelGGL((lm_gemm_kernel<kQ8, true, kQ8 ? 0u : kModelBlocks>), grid,
+                       dim3(kGemmThreads), lds, stream, p);
+  } else {
+    hipLaunchKernelGGL((lm_gemm_kernel<kQ8, true>), grid, dim3(kGemmThreads), lds, stream, p);
+  }
 }
 
-// The narrow GEMM for one configuration: the Q4_0 block loop unrolled whole
-// at the model's width of 896 (28 blocks), a loop otherwise.  (Unrolled, the
-// Q8_0 kernels are scheduled with every block's results live at once: 512
-// registers and scratch memory.)  Workgroups of four waves, two for the Q8_0
-// head with one row tile.  Measured (whole step, us, Q4_0 / Q8_0), four /
-// two / one / eight waves: B = 1 20.2 / 29.9, 21.2 / 29.1, 21.3 / 29.6,
-// 21.1 / 32.1; B = 4 26.5 / 33.2, 27.2 / 33.4, 29.0 / 35.2, 27.5 / 36.1;
-// B = 16 27.5 / 34.8, 28.2 / 33.8, 27.8 / 34.5, 30.2 / 38.9.
-template <bool kQ8, int kRT, int kSets, int kI, bool kFused>
-static void launch_narrow(uint32_t rows, hipStream_t stream, const LmParams& p) {
-  constexpr int kNW = kQ8 && kRT == 1 ? 2 : 4;
-  const dim3 grid((kTilesPerRow + kNW - 1) / kNW, (rows + 16u * kRT - 1) / (16u * kRT));
-  if constexpr (!kQ8) {
-    if (p.cols == kModelBlocks * 32u) {
-      hipLaunchKernelGGL((lm_gemm_narrow_kernel<kQ8, kRT, kSets, kI, kFused, kModelBlocks, kNW>), grid,
-                         dim3(64 * kNW), 0, stream, p);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((lm_gemm_narrow_kernel<kQ8, kRT, kSets, kI, kFused, 0, kNW>), grid,
-                     dim3(64 * kNW), 0, stream, p);
+// The narrow GEMM for one configuration of row groups and result registers.
+template <bool kQ8, int kGroups, int kRegs, bool kFused, int kWaves>
+static void launch_gemm(const LmParams& p, hipStream_t stream) {
+  constexpr uint32_t kTiles = kWaves / kGroups;
+  constexpr uint32_t kRows = 32u * kGroups;
+  const uint32_t blocks = p.cols / 32u;
+  const dim3 grid((kTilesPerRow + kTiles - 1) / kTiles, (p.rows + kRows - 1) / kRows);
+  uint32_t words = kGroups * blocks * 32u + (uint32_t)kWaves * kTailWords;
+  if (kFused) words += blocks * (p.rows + 1u) * 8u;
+  const size_t lds = words * sizeof(float);
+  hipLaunchKernelGGL((lm_gemm_narrow_kernel<kQ8, kGroups, kRegs, kFused, kWaves>), grid, dim3(64 * kWaves),
+                     lds, stream, p);
+}
+
+// Result registers by rows (their epilogue is the work that grows with them),
+// and from 33 rows two row groups per workgroup.  Workgroups of four waves, two
+// for the Q8_0 head with one row group (one row 35.0 -> 33.2 us, 16 rows 42.0
+// -> 38.8: 594 workgroups of four leave some CUs three and others two).
+// Measured per step (us) against one or two row tiles of 16 rows on
+// v_mfma_i32_16x16x32_i8 with the scales loaded beside the operands:
+//   rows      1     4     8     16    24    32    40    64
+//   Q4_0      20.1  26.2  27.3  27.8  38.0  38.3  55.8  56.9
+//     now     20.5  21.9  22.7  25.4  28.0  31.4  41.5  43.2
+//   Q8_0      33.1  35.8  37.5  38.7  57.9  58.8  66.8  70.6
+//     now     31.4  34.7  35.4  37.5  40.1  42.4  51.3  54.6
+template <bool kQ8>
+static void launch_gemm_rows(const LmParams& p, hipStream_t stream) {
+  if (p.rows > kNarrowRows) return launch_gemm_wide<kQ8>(p, stream);
+  constexpr int kW = kQ8 ? 2 : 4;
+  if (p.rows == 1) return launch_gemm<kQ8, 1, 1, true, kW>(p, stream);
+  if (p.rows == 2) return launch_gemm<kQ8, 1, 2, true, kW>(p, stream);
+  if (p.fused_quant) return launch_gemm<kQ8, 1, 4, true, kW>(p, stream);
+  if (p.rows <= 8) return launch_gemm<kQ8, 1, 4, false, kW>(p, stream);
+  if (p.rows <= 16) return launch_gemm<kQ8, 1, 8, false, kW>(p, stream);
+  if (p.rows <= 24) return launch_gemm<kQ8, 1, 12, false, kW>(p, stream);
+  if (p.rows <= 32) return launch_gemm<kQ8, 1, 16, false, kW>(p, stream);
+  return launch_gemm<kQ8, 2, 16, false, 4>(p, stream);
 }
 
 hipError_t launch_lm_sample(const LmParams& p, const RowParams& rp, hipStream_t stream) {
@@ -2115,64 +2345,10 @@ hipError_t launch_lm_sample(const LmParams& p, const RowParams& rp, hipStream_t 
     hipLaunchKernelGGL(lm_quant_kernel, dim3((pairs + kBlockThreads / 8u - 1) / (kBlockThreads / 8u)),
                        dim3(kBlockThreads), 0, stream, p);
   }
-  if (p.rows <= kNarrowRows) {
-    // Loads one block ahead.  Measured (whole step, HIP events, us) with the
-    // Q4_0 block loop unrolled at width 896, one / two / three / five / seven
-    // blocks ahead: B = 1 19.5 / 20.5 / 20.7 / 22.8 / 23.0, B = 4 26.3 / 26.3
-    // / 27.8 / 28.2 / 36.8, B = 32 39.7 / 40.7 / 42.2 / 43.2 / 51.7; two row
-    // tiles (B = 64) 59.2 / 60.2 / 60.4 / 76.4 / 79.2.  Splitting a tile's
-    // 28 blocks over two or four waves (each keeping its terms until the
-    // previous part's running totals arrive through LDS, so the sums stay in
-    // block order) was slower: B = 1 22.6-25.4 us.
-    const uint32_t rt = p.rows <= 32u ? 1u : 2u;
-    if (p.q8) {
-      if (p.rows == 1)
-        launch_narrow<true, 1, 2, 1, true>(p.rows, stream, p);
-      else if (p.rows == 2)
-        launch_narrow<true, 1, 2, 2, true>(p.rows, stream, p);
-      else if (p.fused_quant)
-        launch_narrow<true, 1, 2, 4, true>(p.rows, stream, p);
-      else if (rt == 1)
-        launch_narrow<true, 1, 2, 4, false>(p.rows, stream, p);
-      else
-        launch_narrow<true, 2, 2, 4, false>(p.rows, stream, p);
-    } else {
-      if (p.rows == 1)
-        launch_narrow<false, 1, 2, 1, true>(p.rows, stream, p);
-      else if (p.rows == 2)
-        launch_narrow<false, 1, 2, 2, true>(p.rows, stream, p);
-      else if (p.fused_quant)
-        launch_narrow<false, 1, 2, 4, true>(p.rows, stream, p);
-      else if (rt == 1)
-        launch_narrow<false, 1, 2, 4, false>(p.rows, stream, p);
-      else
-        launch_narrow<false, 2, 2, 4, false>(p.rows, stream, p);
-    }
-  } else {
-    const dim3 gemm_grid(kTilesPerRow, (p.rows_pad + kRowsPerGroup - 1) / kRowsPerGroup);
-    const size_t lds = gemm_lds_bytes(p.cols);
-    const bool model_width = p.cols == kModelBlocks * 32u;  // the Q4_0 loop unrolled whole
-    if (p.logits == nullptr) {  // one pass: tile and second words, no logits
-      if (p.q8)
-        hipLaunchKernelGGL((lm_gemm_kernel<true, false>), gemm_grid, dim3(kGemmThreads), lds,
-                           stream, p);
-      else if (model_width)
-        hipLaunchKernelGGL((lm_gemm_kernel<false, false, kModelBlocks>), gemm_grid,
-                           dim3(kGemmThreads), lds, stream, p);
-      else
-        hipLaunchKernelGGL((lm_gemm_kernel<false, false>), gemm_grid, dim3(kGemmThreads), lds,
-                           stream, p);
-    } else if (p.q8) {
-      hipLaunchKernelGGL((lm_gemm_kernel<true, true>), gemm_grid, dim3(kGemmThreads), lds, stream,
-                         p);
-    } else if (model_width) {
-      hipLaunchKernelGGL((lm_gemm_kernel<false, true, kModelBlocks>), gemm_grid,
-                         dim3(kGemmThreads), lds, stream, p);
-    } else {
-      hipLaunchKernelGGL((lm_gemm_kernel<false, true>), gemm_grid, dim3(kGemmThreads), lds,
-                         stream, p);
-    }
-  }
+  if (p.q8)
+    launch_gemm_rows<true>(p, stream);
+  else
+    launch_gemm_rows<false>(p, stream);
   if (p.logits == nullptr) {  // one pass: no logits kept, the selection recomputes tiles
     if (p.q8)
       hipLaunchKernelGGL(lm_select_kernel<kRecomputeQ8>, dim3(p.rows), dim3(kSelectThreads), 0,

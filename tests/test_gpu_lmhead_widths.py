@@ -78,3 +78,36 @@ def test_logits_and_draws_at_each_width(smp, q8, cols):
                                        np.zeros(rows, np.uint32), r24, threads=4)
         gtok = token.cpu().numpy().view(np.uint32)
         assert (gtok == rtok).all(), (cols, rows)
+
+
+@pytest.mark.parametrize("q8", [False, True], ids=["q4_0", "q8_0"])
+@pytest.mark.parametrize("cols", [32, 96, 128])
+def test_narrow_head_either_side_of_every_row_count_it_branches_on(smp, q8, cols):
+    """One row to 65: the narrow kernel keeps 1, 2, 4, 8, 12 or 16 result
+    registers by the rows, in one row group or two, and 65 rows take the wide
+    kernel.  Odd block counts carry an infinite scale in one Q4_0 tile, which
+    is computed again.  Every value is defined bit for bit, so it must agree."""
+    import torch
+
+    head = make_head(cols, q8, seed=cols + (2000 if q8 else 0))
+    packed = smp.pack_lmhead(torch.from_numpy(head).to("cuda:0"), q8=q8, cols=cols)
+    rng = np.random.default_rng(cols + 7)
+    hidden = rng.standard_normal((65, cols)).astype(np.float32)
+    rlog = o.lmhead_logits(hidden, head, V, cols, threads=16, q8=q8)
+    rnan = np.isnan(rlog.view(np.float32))
+    for rows in (1, 2, 3, 4, 5, 8, 9, 16, 17, 24, 25, 32, 33, 64, 65):
+        r24 = (np.arange(rows, dtype=np.uint32) * 7919 + 3) & 0xFFFFFF
+        token = torch.empty(rows, dtype=torch.int32, device="cuda:0")
+        logits = torch.full((rows + 1, V), -1, dtype=torch.int32, device="cuda:0")
+        smp.lmhead_sample(packed, to_dev(hidden[:rows]), to_dev(r24), token=token,
+                          logits=logits, cols=cols, q8=q8)
+        torch.cuda.synchronize()
+        glog = logits.cpu().numpy().view(np.uint32)
+        assert (glog[rows] == 0xFFFFFFFF).all(), (cols, rows)  # nothing past the last row
+        gnan = np.isnan(glog[:rows].view(np.float32))
+        assert (gnan == rnan[:rows]).all(), (cols, rows)
+        bad = np.argwhere((glog[:rows] != rlog[:rows]) & ~rnan[:rows])
+        assert bad.size == 0, (cols, rows, bad[:5])
+        rtok, _, _, _ = o.sample_batch(rlog[:rows], np.zeros((rows, 1), np.uint32),
+                                       np.zeros(rows, np.uint32), r24, threads=4)
+        assert (token.cpu().numpy().view(np.uint32) == rtok).all(), (cols, rows)
