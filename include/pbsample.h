@@ -417,7 +417,7 @@ uint32_t pb_decode_settle(pb_sampling_state *states, const pb_sampling_state *sa
                           const uint32_t *state_before, const uint32_t *tokens, uint32_t rows);
 
 /* Batches of up to PB_TILE_SELECT_ROWS rows under the automatic plan (and
- * without a `seen` exclusion) are sampled through per-tile summaries of the
+ * without a `seen` scratch that is not 16-byte aligned) are sampled through per-tile summaries of the
  * logits and the fused LM head's selection kernel; larger batches, and every
  * batch under a forced slice plan, stream each row in slices. */
 #define PB_TILE_SELECT_ROWS 192u

@@ -1486,7 +1486,9 @@ __device__ __forceinline__ uint64_t tile_bound(uint64_t key) {
 // read.  Error rows: the lowest tile flagged kNonFiniteTile holds the first
 // non-finite logit (NONFINITE_OUTPUT, which takes precedence), else the first
 // history id >= vocab (TOKEN_ID).  The row is finished with finalize_row.
-template <int kSrc>
+// kExcl: the ids already set in the row's `seen` scratch (rp.excl, 16-byte
+// aligned) are taken out of the bitmap once it is built.
+template <int kSrc, bool kExcl = false>
 __global__ __launch_bounds__(kSelectThreads) void lm_select_kernel(LmParams p, RowParams rp) {
   constexpr bool kRecompute = kSrc != kFromLogits;
   __shared__ __align__(16) uint32_t bm[kWordsPerRow];
@@ -1567,6 +1569,16 @@ __global__ __launch_bounds__(kSelectThreads) void lm_select_kernel(LmParams p, R
       act_word = reinterpret_cast<const uint32_t*>(
           p.act_q + ((size_t)(tid >> 3) * p.rows_pad + row) * 32u)[tid & 7u];
     if (tid < blocks) act_scale = p.act_s[(size_t)tid * p.rows_pad + row];
+  }
+  // the `seen` scratch, requested with the rest
+  constexpr uint32_t kSeenV4 = kWordsPerRow / 4u;
+  constexpr uint32_t kSeenPer = kExcl ? (kSeenV4 + kSelectThreads - 1u) / kSelectThreads : 1u;
+  static_assert(PB_SEEN_BYTES == kWordsPerRow * 4u, "a scratch row is the bitmap's size");
+  v4u ex[kSeenPer];
+  if constexpr (kExcl) {
+    const v4u* seen = reinterpret_cast<const v4u*>(rp.excl + (size_t)row * PB_SEEN_BYTES);
+#pragma unroll
+    for (uint32_t u = 0; u < kSeenPer; ++u) ex[u] = seen[min(tid + u * kSelectThreads, kSeenV4 - 1u)];
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -2001,6 +2013,17 @@ __global__ __launch_bounds__(kSelectThreads) void lm_select_kernel(LmParams p, R
     if (lane == 0 && my_bad != kNone) atomicMin(&bad_hist, my_bad);
   }
   __syncthreads();  // (3) the bitmap, the first-round lists and the errors are done
+  if constexpr (kExcl) {
+#pragma unroll
+    for (uint32_t u = 0; u < kSeenPer; ++u) {
+      const uint32_t i = tid + u * kSelectThreads;
+      if (i < kSeenV4) {
+        v4u* word = &reinterpret_cast<v4u*>(bm)[i];
+        *word = *word & ~ex[u];
+      }
+    }
+    __syncthreads();
+  }
   recompute_listed();  // (recompute mode: the first round's listed tiles)
 
   // ---- wave 0: errors, then the first round's candidates ----
@@ -2397,8 +2420,12 @@ hipError_t launch_tile_select(const LmParams& p, const RowParams& rp, hipStream_
     sp.logits = p.logits_copy;
     sp.logits_copy = nullptr;
   }
-  hipLaunchKernelGGL(lm_select_kernel<kFromLogits>, dim3(p.rows), dim3(kSelectThreads), 0, stream,
-                     sp, rp);
+  if (rp.excl != nullptr)
+    hipLaunchKernelGGL((lm_select_kernel<kFromLogits, true>), dim3(p.rows), dim3(kSelectThreads), 0,
+                       stream, sp, rp);
+  else
+    hipLaunchKernelGGL(lm_select_kernel<kFromLogits>, dim3(p.rows), dim3(kSelectThreads), 0, stream,
+                       sp, rp);
   return hipGetLastError();
 }
 

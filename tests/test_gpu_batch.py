@@ -202,6 +202,48 @@ def test_inplace_variant_penalises_like_the_reference(sampler):
     assert not seen.cpu().numpy().any()
 
 
+@pytest.mark.parametrize("rows, shift, hist_ld", [(1, 0, 3), (3, 0, 300), (4, 4, 301), (40, 0, 2049),
+                                                  (192, 0, 4100), (193, 0, 512)])
+def test_inplace_with_a_dirty_seen_scratch(sampler, rows, shift, hist_ld):
+    """Either side of the tile selection's row limit, a scratch that cannot be
+    read 16 bytes at a time (the slice plan), histories shorter than a
+    thread's batch and longer than several: tokens, logits and scratch are the
+    oracle's, word for word."""
+    import torch
+
+    sampler.set_segments(0)
+    rng = np.random.default_rng(rows + hist_ld)
+    logits = workloads.boosted_normal(rng, rows)
+    lengths = rng.integers(0, hist_ld + 1, rows).astype(np.uint32)
+    lengths[0] = hist_ld
+    hist = workloads.zipf_history(rng, lengths, hist_ld)
+    if rows > 3:
+        logits[2, 5] = np.inf   # fails: logits, scratch and draw untouched
+    if rows > 4:
+        hist[3, 0] = V          # fails when its history is not empty
+    seen = (rng.random((rows, s.SEEN_BYTES)) < 0.02).astype(np.uint8) * np.uint8(0x11)
+    # the scratch holds some of the history's own ids (Zipf: the low ones)
+    seen[:, :4] |= rng.integers(0, 256, (rows, 4), dtype=np.uint8)
+    seeds = np.arange(rows, dtype=np.uint64) + np.uint64(77)
+    r24 = workloads.next_24_stream(seeds)
+    dl = to_dev(logits)
+    raw = torch.zeros(rows * s.SEEN_BYTES + 16, dtype=torch.uint8, device="cuda:0")
+    raw[shift:shift + seen.size] = torch.from_numpy(seen.reshape(-1)).to("cuda:0")
+    token = torch.empty(rows, dtype=torch.int32, device="cuda:0")
+    sampler.sample(dl, to_dev(r24), to_dev(hist), to_dev(lengths), token=token, inplace=True,
+                   seen=raw.data_ptr() + shift)
+    torch.cuda.synchronize()
+    got = dl.cpu().numpy().view(np.uint32)
+    gseen = raw.cpu().numpy()[shift:shift + seen.size].reshape(rows, -1)
+    gtok = token.cpu().numpy().view(np.uint32)
+    for r in range(rows):
+        ref, rseen = logits[r].view(np.uint32).copy(), seen[r].copy()
+        st, rt, _ = o.sample_token_with_repetition(ref, hist[r, :lengths[r]], rseen,
+                                                   o.SamplingState(int(seeds[r])))
+        assert gtok[r] == (rt if st == 0 else s.NO_TOKEN), r
+        assert (got[r] == ref).all() and (gseen[r] == rseen).all(), r
+
+
 def test_rows_are_independent_of_batch_neighbours(sampler):
     w = workloads.make("small", rows=64)
     full = run_gpu(sampler, w)
