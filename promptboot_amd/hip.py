@@ -14,6 +14,7 @@ valid across both; otherwise the dynamic loader finds /opt/rocm's.
 from __future__ import annotations
 
 import ctypes
+import math
 
 import numpy as np
 
@@ -178,6 +179,18 @@ class DeviceArray:
     def zeros(cls, shape, dtype=np.uint32) -> "DeviceArray":
         return cls.from_numpy(np.zeros(shape, dtype))
 
+    def part(self, start: int, shape) -> "DeviceArray":
+        """A view of this buffer's elements from `start` on, in its dtype; it
+        keeps the buffer alive and frees nothing itself."""
+        d = DeviceArray.__new__(DeviceArray)
+        d.shape = tuple(int(x) for x in (shape if np.iterable(shape) else (shape,)))
+        d.dtype, d._base = self.dtype, self
+        d.nbytes = math.prod(d.shape) * d.dtype.itemsize
+        if start < 0 or start * d.dtype.itemsize + d.nbytes > self.nbytes:
+            raise ValueError(f"elements {start} .. of shape {d.shape} lie outside the buffer")
+        d._ptr = self._ptr + start * d.dtype.itemsize
+        return d
+
     def data_ptr(self) -> int:
         return self._ptr
 
@@ -210,7 +223,9 @@ class DeviceArray:
                                                             D2D, stream_handle(stream)))
 
     def free(self) -> None:
-        if self._ptr:
+        if getattr(self, "_base", None) is not None:  # a view
+            self._ptr, self._base = 0, None
+        elif self._ptr:
             runtime().hipFree(self._ptr)
             self._ptr = 0
 

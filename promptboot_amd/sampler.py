@@ -27,6 +27,7 @@ the import fails.
 from __future__ import annotations
 
 import ctypes
+import math
 import pathlib
 
 import numpy as np
@@ -321,14 +322,14 @@ def _dev(x, name: str, *, itemsize: int = 4, rows: int | None = None,
         raise ValueError(f"{name} must have {ndim} dimensions, has shape {shape}")
     if rows is not None:
         need = rows * (row_elems if row_elems is not None else 1)
-        have = int(np.prod(shape, dtype=np.int64))
+        have = math.prod(shape)
         if have < need:
             raise ValueError(f"{name} holds {have} elements, {need} needed for {rows} rows")
     return vp(x.data_ptr())
 
 
 def _nbytes(x) -> int:
-    return int(np.prod(_shape(x), dtype=np.int64)) * _itemsize(x)
+    return math.prod(_shape(x)) * _itemsize(x)
 
 
 class BatchSampler:
@@ -556,13 +557,18 @@ class DecodeBatch:
         dev = hip.DeviceArray.from_numpy
         self.hist, self.hist_len, self.max_len = dev(hist), dev(lens), dev(max_len)
         self.row_state_host = np.where(lens < max_len, ROW_ACTIVE, ROW_LIMIT).astype(np.uint32)
-        self.row_state = dev(self.row_state_host)
+        # The uniforms, tokens and row states are one device block with one
+        # pinned copy: a step sends the first third and fetches the rest, one
+        # stream-ordered copy each way.
+        self._io = hip.DeviceArray(3 * self.rows, np.uint32)
+        self._host = hip.PinnedArray(3 * self.rows, np.uint32)
+        self.r24, self.token, self.row_state = (
+            self._io.part(k * self.rows, self.rows) for k in range(3))
+        self.row_state.upload(self.row_state_host)
         self.states = (_State * self.rows)()
         for r, seed in enumerate(seeds):
             lib().pb_sampling_state_new(ctypes.byref(self.states[r]), int(seed) & (2**64 - 1))
         self._saved = (_State * self.rows)()
-        self.r24 = hip.DeviceArray(self.rows, np.uint32)
-        self.token = hip.DeviceArray(self.rows, np.uint32)
         self.err = hip.DeviceArray((self.rows, ERROR_DTYPE.itemsize // 4), np.uint32)
 
     def close(self):
@@ -573,25 +579,31 @@ class DecodeBatch:
     def active(self) -> bool:
         return bool((self.row_state_host == ROW_ACTIVE).any())
 
-    def _draw(self):
-        r24 = np.zeros(self.rows, np.uint32)
+    def _draw(self, stream):
+        """One uniform per active row, on its way to the device on `stream`."""
         before = self.row_state_host.copy()
-        lib().pb_decode_draw(self.states, before.ctypes.data_as(vp), self.rows,
-                             r24.ctypes.data_as(vp), self._saved)
-        self.r24.upload(r24)
+        # whatever produces the step's input has run, and no copy of an earlier
+        # step still reads the pinned buffer
+        hip.synchronize()
+        lib().pb_decode_draw(self.states, before.ctypes.data, self.rows, self._host.data_ptr(),
+                             self._saved)
+        hip.copy_async(self._io.data_ptr(), self._host.data_ptr(), 4 * self.rows, hip.H2D, stream)
         return before
 
     def _undraw(self):
         for r in range(self.rows):
             self.states[r] = self._saved[r]
 
-    def _settle(self, before):
-        after = self.row_state.numpy()
-        tokens = self.token.numpy()
-        lib().pb_decode_settle(self.states, self._saved, before.ctypes.data_as(vp),
-                               tokens.ctypes.data_as(vp), self.rows)
+    def _settle(self, before, stream):
+        out = 4 * self.rows
+        hip.copy_async(self._host.data_ptr() + out, self._io.data_ptr() + out, 2 * out, hip.D2H,
+                       stream)
+        hip.synchronize()
+        tokens, after = self._host.array[self.rows:].reshape(2, self.rows).copy()
+        lib().pb_decode_settle(self.states, self._saved, before.ctypes.data, tokens.ctypes.data,
+                               self.rows)
         self.row_state_host = after
-        return tokens.copy()
+        return tokens
 
     def _ptrs(self):
         return (vp(self.hist.data_ptr()), self.hist_ld, vp(self.hist_len.data_ptr()),
@@ -607,7 +619,7 @@ class DecodeBatch:
         if rows != self.rows:
             raise ValueError(f"logits have {rows} rows, the batch has {self.rows}")
         lp = _dev(logits, "logits", ndim=2)
-        before = self._draw()
+        before = self._draw(stream)
         e = _Error()
         try:
             st = lib().pb_decode_step(self.sampler._ctx, lp, VOCAB, ld, self.rows, *self._ptrs(),
@@ -616,7 +628,7 @@ class DecodeBatch:
         except Exception:
             self._undraw()
             raise
-        return self._settle(before)
+        return self._settle(before, stream)
 
     def lmhead_step(self, packed, hidden, cols: int | None = None, stream=None,
                     q8: bool = False) -> np.ndarray:
@@ -627,7 +639,7 @@ class DecodeBatch:
             raise ValueError(f"hidden has {rows} rows, the batch has {self.rows}")
         self.sampler._ensure(rows, width)
         pp, hp = _dev(packed, "packed", itemsize=1), _dev(hidden, "hidden", ndim=2)
-        before = self._draw()
+        before = self._draw(stream)
         fn = lib().pb_lmhead_q8_decode_step if q8 else lib().pb_lmhead_decode_step
         e = _Error()
         try:
@@ -638,7 +650,7 @@ class DecodeBatch:
         except Exception:
             self._undraw()
             raise
-        return self._settle(before)
+        return self._settle(before, stream)
 
     def contexts(self) -> list[np.ndarray]:
         h = self.hist.numpy()

@@ -247,3 +247,19 @@ def test_random_decode_loops_match_the_oracle(seed, n):
     nan_at = {int(r): int(rng.integers(0, 8)) for r in rng.choice(n, max(1, n // 25), replace=False)}
     segments = int(rng.choice([0, 0, 1, 3]))
     run_lockstep(prompts, seeds, limits, eos_after, eos_ids, nan_at, 14, segments)
+
+
+def test_parts_of_a_device_buffer_share_its_memory():
+    """The step's uniforms, tokens and row states are parts of one buffer."""
+    from promptboot_amd import hip
+
+    block = hip.DeviceArray.zeros(9, np.uint32)
+    first, last = block.part(0, 3), block.part(6, (1, 3))
+    last.upload(np.array([7, 8, 9], np.uint32))
+    assert block.numpy().tolist() == [0] * 6 + [7, 8, 9]
+    assert last.numpy().tolist() == [[7, 8, 9]] and not first.numpy().any()
+    first.free()  # a part owns nothing
+    assert block.numpy().tolist() == [0] * 6 + [7, 8, 9]
+    for start, n in ((7, 3), (-1, 2), (9, 1)):
+        with pytest.raises(ValueError):
+            block.part(start, n)
