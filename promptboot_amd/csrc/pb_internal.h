@@ -79,7 +79,7 @@ struct LmParams {
   uint32_t* tilesec;        // rows x 2,374 second words (narrow GEMM and one pass, else null):
                             // a bound above every other logit's order word of the tile
                             // (a multiple of 64) plus the maximum's index in the tile
-  // tile_words_kernel only (null / 0 otherwise): the logits it reads are also
+  // tile_words_copy_kernel only (null / 0 otherwise): the logits it reads are also
   // stored at logits_copy (same ld), and stage_v4 16-byte groups are copied
   // from stage_src to stage_dst on the way, so that logits and small inputs
   // read from pinned host memory reach the device in the same launch.

@@ -380,6 +380,67 @@ __device__ __forceinline__ uint32_t tile_second_word(const uint32_t (&ow)[4], ui
   return (((other >> 6) + 1u) << 6) | (first & kSecondIndexMask);
 }
 
+// ---- a tile's words from LDS, four lanes a tile ----
+// `mine` points at the lane's 16 of the tile's 64 logits (ids 16 qd ..), 16-byte
+// aligned; the four lanes of a quad hold one tile.  The largest of each four
+// ids, the two largest of those four maxima, then the largest one's group read
+// again for its place and second value, and a reduction over four lanes:
+// about 50 vector instructions for 16 tiles, against 180 with one 16-lane
+// reduction for every four.  A tie at the maximum, in a group or across, makes
+// the bound on the other logits reach the tile word.  The sign of a zero
+// maximum is not kept: the selection reads a tile whose word is the order word
+// of zero.
+constexpr uint32_t kTailStride = 68;  // words of a tile's row in LDS: 16-byte reads meet no bank twice
+constexpr uint32_t kTailWords = 16 * kTailStride;
+__device__ __forceinline__ void four_lane_words(const float* mine, uint32_t qd, uint32_t& tile_word,
+                                                uint32_t& second) {
+  v4f v[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const v4f*>(mine + 4 * k);
+  float probe = 0.0f;
+  float gm[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) probe = __builtin_fmaf(v[k][c], 0.0f, probe);
+    // (only used when every value is finite: no quietening of NaN operands)
+    __asm__("v_max3_f32 %0, %1, %2, %3\n\tv_max_f32 %0, %0, %4"
+            : "=&v"(gm[k])
+            : "v"(v[k].x), "v"(v[k].y), "v"(v[k].z), "v"(v[k].w));
+  }
+  float m3, md, lo, m, sg;
+  __asm__("v_max3_f32 %0, %1, %2, %3" : "=v"(m3) : "v"(gm[0]), "v"(gm[1]), "v"(gm[2]));
+  __asm__("v_med3_f32 %0, %1, %2, %3" : "=v"(md) : "v"(gm[0]), "v"(gm[1]), "v"(gm[2]));
+  __asm__("v_min_f32 %0, %1, %2" : "=v"(lo) : "v"(m3), "v"(gm[3]));
+  __asm__("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(m3), "v"(gm[3]));
+  __asm__("v_max_f32 %0, %1, %2" : "=v"(sg) : "v"(md), "v"(lo));
+  uint32_t k = gm[2] == m ? 8u : 12u;
+  k = gm[1] == m ? 4u : k;
+  k = gm[0] == m ? 0u : k;
+  const v4f w = *reinterpret_cast<const v4f*>(mine + k);
+  float s2;
+  __asm__("v_max3_f32 %0, %1, %2, %3" : "=v"(m3) : "v"(w.x), "v"(w.y), "v"(w.z));
+  __asm__("v_med3_f32 %0, %1, %2, %3" : "=v"(md) : "v"(w.x), "v"(w.y), "v"(w.z));
+  __asm__("v_min_f32 %0, %1, %2" : "=v"(lo) : "v"(m3), "v"(w.w));
+  __asm__("v_max3_f32 %0, %1, %2, %3" : "=v"(s2) : "v"(md), "v"(lo), "v"(sg));
+  uint32_t c = w.z == m ? 2u : 3u;
+  c = w.y == m ? 1u : c;
+  c = w.x == m ? 0u : c;
+  const uint32_t at = 16u * qd + k + c;
+  const uint32_t o = probe != probe ? kNonFiniteTile : order_word(m);
+  // over the row's four lanes
+  uint32_t word = max(o, dpp_or_zero<0xB1>(o));
+  word = max(word, dpp_or_zero<0x4E>(word));
+  uint32_t idx = o == word ? at : 0xffu;
+  idx = min(idx, dpp_or_zero<0xB1>(idx));
+  idx = min(idx, dpp_or_zero<0x4E>(idx));
+  uint32_t other = at == idx ? order_word(s2) : o;
+  other = max(other, dpp_or_zero<0xB1>(other));
+  other = max(other, dpp_or_zero<0x4E>(other));
+  tile_word = word;
+  second = ((other & ~kSecondIndexMask) + 64u) | idx;
+}
+
 // ---- a wide wave's results for one 64-id tile, logits kept ----
 // total[rt][c][i] is row base_row + lane_row + 16 rt + i, id 64 tile + 4n + c,
 // where base_row is the first row of the wave's group of group_rows rows and
@@ -852,8 +913,6 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
 // a group or across, makes the bound on the other logits reach the tile
 // word.  The sign of a zero maximum is not kept: the selection reads a tile
 // whose word is the order word of zero.
-constexpr uint32_t kTailStride = 68;
-constexpr uint32_t kTailWords = 16 * kTailStride;
 template <int kRegs>
 __device__ __forceinline__ void write_tile(const LmParams& p, const v4f (&total)[2][(kRegs + 3) / 4],
                                            uint32_t base_row, uint32_t group_rows,
@@ -919,53 +978,12 @@ __device__ __forceinline__ void write_tile(const LmParams& p, const v4f (&total)
                                 2u * j) = v2f{total[0][i / 4][i % 4], total[1][i / 4][i % 4]};
     }
     __builtin_amdgcn_wave_barrier();
-    v4f v[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const v4f*>(mine + 4 * k);
-    float probe = 0.0f;
-    float gm[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) probe = __builtin_fmaf(v[k][c], 0.0f, probe);
-      // (only used when every value is finite: no quietening of NaN operands)
-      __asm__("v_max3_f32 %0, %1, %2, %3\n\tv_max_f32 %0, %0, %4"
-              : "=&v"(gm[k])
-              : "v"(v[k].x), "v"(v[k].y), "v"(v[k].z), "v"(v[k].w));
-    }
-    float m3, md, lo, m, sg;
-    __asm__("v_max3_f32 %0, %1, %2, %3" : "=v"(m3) : "v"(gm[0]), "v"(gm[1]), "v"(gm[2]));
-    __asm__("v_med3_f32 %0, %1, %2, %3" : "=v"(md) : "v"(gm[0]), "v"(gm[1]), "v"(gm[2]));
-    __asm__("v_min_f32 %0, %1, %2" : "=v"(lo) : "v"(m3), "v"(gm[3]));
-    __asm__("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(m3), "v"(gm[3]));
-    __asm__("v_max_f32 %0, %1, %2" : "=v"(sg) : "v"(md), "v"(lo));
-    uint32_t k = gm[2] == m ? 8u : 12u;
-    k = gm[1] == m ? 4u : k;
-    k = gm[0] == m ? 0u : k;
-    const v4f w = *reinterpret_cast<const v4f*>(mine + k);
-    float s2;
-    __asm__("v_max3_f32 %0, %1, %2, %3" : "=v"(m3) : "v"(w.x), "v"(w.y), "v"(w.z));
-    __asm__("v_med3_f32 %0, %1, %2, %3" : "=v"(md) : "v"(w.x), "v"(w.y), "v"(w.z));
-    __asm__("v_min_f32 %0, %1, %2" : "=v"(lo) : "v"(m3), "v"(w.w));
-    __asm__("v_max3_f32 %0, %1, %2, %3" : "=v"(s2) : "v"(md), "v"(lo), "v"(sg));
-    uint32_t c = w.z == m ? 2u : 3u;
-    c = w.y == m ? 1u : c;
-    c = w.x == m ? 0u : c;
-    const uint32_t at = 16u * qd + k + c;
-    const uint32_t o = probe != probe ? kNonFiniteTile : order_word(m);
-    // over the row's four lanes
-    uint32_t word = max(o, dpp_or_zero<0xB1>(o));
-    word = max(word, dpp_or_zero<0x4E>(word));
-    uint32_t idx = o == word ? at : 0xffu;
-    idx = min(idx, dpp_or_zero<0xB1>(idx));
-    idx = min(idx, dpp_or_zero<0x4E>(idx));
-    uint32_t other = at == idx ? order_word(s2) : o;
-    other = max(other, dpp_or_zero<0xB1>(other));
-    other = max(other, dpp_or_zero<0x4E>(other));
+    uint32_t word, second;
+    four_lane_words(mine, qd, word, second);
     if (qd == 0u) {
       const uint32_t off = ((wave_row + 16u * (uint32_t)half + (lane >> 2)) * kTilesPerRow + tile) * 4u;
       __builtin_amdgcn_raw_buffer_store_b32(word, tm, off, 0, 0);
-      __builtin_amdgcn_raw_buffer_store_b32(((other & ~kSecondIndexMask) + 64u) | idx, ts, off, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b32(second, ts, off, 0, 0);
     }
     __builtin_amdgcn_wave_barrier();
   };
@@ -1326,19 +1344,18 @@ __device__ __forceinline__ uint32_t collect_range(uint64_t* cand, const uint64_t
   return uniform(count);
 }
 
-// ---- tile words of given logits (the batched sampler's small batches) ----
+// ---- tile words of a single-row drop-in's logits ----
 // The same tile and second words as the narrow GEMM writes, from logits in
-// memory: one 16-lane row per (row, 64-id tile), lane n reading ids
-// 4n .. 4n+3 of the tile (one 16-byte load each, read once).  A workgroup
-// takes 16 x kLoads consecutive tiles of one row, each 16-lane row kLoads of
-// them (tiles g, g + 16, ...: every load instruction covers 16 whole tiles),
-// all loads in flight together; the grid's y runs over the rows.  For a
-// single-row drop-in the logits are in mapped pinned host memory: the launch
-// also stores them at logits_copy and copies the staged scalars and history,
-// so that the selection reads device memory (on MI355X the PCIe read of the
-// 608 KB row takes about 15 us, at 128 to 1,024 threads per workgroup alike).
-template <uint32_t kLoads>
-__global__ __launch_bounds__(256) void tile_words_kernel(LmParams p) {
+// mapped pinned host memory: one 16-lane row per 64-id tile, lane n reading
+// ids 4n .. 4n+3 of the tile (one 16-byte load each, read once).  A workgroup
+// takes 64 consecutive tiles, each 16-lane row four of them (tiles g, g + 16,
+// ...: every load instruction covers 16 whole tiles), all loads in flight
+// together.  The launch also stores the logits at logits_copy and copies the
+// staged scalars and history, so that the selection reads device memory (on
+// MI355X the PCIe read of the 608 KB row takes about 15 us, at 128 to 1,024
+// threads per workgroup and two to eight loads per thread alike).
+__global__ __launch_bounds__(256) void tile_words_copy_kernel(LmParams p) {
+  constexpr uint32_t kLoads = 4;
   constexpr uint32_t kTilesPerGroup = 16u * kLoads;
   const uint32_t n = threadIdx.x & 15u;
   const uint32_t g = threadIdx.x >> 4;
@@ -1358,10 +1375,7 @@ __global__ __launch_bounds__(256) void tile_words_kernel(LmParams p) {
     reinterpret_cast<v4u*>(p.stage_dst)[i] = reinterpret_cast<const v4u*>(p.stage_src)[i];
   // Every word is computed before anything is stored: the wait for a load
   // issued before a store also waits for the store (one counter for both on
-  // gfx950), and under the stream's read traffic a store's acknowledgement
-  // takes microseconds.  Storing the first tile's words before the second
-  // load was used made the B = 64 step 0.9 us longer (16.4 against 15.5 us
-  // per step cold, wall).
+  // gfx950).
   uint32_t word[kLoads], sec[kLoads];
 #pragma unroll
   for (uint32_t k = 0; k < kLoads; ++k) {
@@ -1373,13 +1387,58 @@ __global__ __launch_bounds__(256) void tile_words_kernel(LmParams p) {
 #pragma unroll
   for (uint32_t k = 0; k < kLoads; ++k) {
     const uint32_t tile = blockIdx.x * kTilesPerGroup + g + 16u * k;
-    if (p.logits_copy != nullptr && tile < kTilesPerRow)
+    if (tile < kTilesPerRow)
       *reinterpret_cast<v4u*>(p.logits_copy + (size_t)row * p.logits_ld + tile * kTileIds + 4u * n) =
           x[k];
     if (n == 0u && tile < kTilesPerRow) {
       p.tilemax[(size_t)row * kTilesPerRow + tile] = word[k];
       p.tilesec[(size_t)row * kTilesPerRow + tile] = sec[k];
     }
+  }
+}
+
+// ---- tile words of given logits (the batched sampler's small batches) ----
+// The same words, from logits in HBM: a wave reads 16 consecutive tiles of a
+// row (four whole-line loads per lane, in flight together), stores them to its
+// own LDS and reduces them four lanes a tile (four_lane_words); the grid's y
+// runs over the rows.  Bound by the read from about 100 rows up, below by the
+// chain of one read, one reduction and one store.  Steps of the sampler (us)
+// against one 16-lane row per tile and two tiles per row of lanes, which
+// spends 180 vector instructions on 16 tiles instead of 50:
+//   rows      1    4    16    32    48    64    100   180
+//             7.8  8.4  10.1  11.8  13.3  14.9  18.3  26.6
+//   now       7.8  8.1   9.7  10.8  12.4  13.9  17.4  26.5
+// Workgroups of two waves: four measured 0.1-0.2 us more, one 0.8 us more at
+// 64 rows and 0.1 less up to three rows.  (About 2,048 workgroups in grid-stride order over the batch, three
+// loads ahead, were 5-10 us slower: few waves, each behind its own chain.)
+template <uint32_t kWaves>
+__global__ __launch_bounds__(64 * kWaves) void tile_words_kernel(LmParams p) {
+  __shared__ __align__(16) float turn[kWaves][kTailWords];
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = threadIdx.x >> 6;
+  const uint32_t n = lane & 15u;
+  const uint32_t row = blockIdx.y;
+  const uint32_t first = (blockIdx.x * kWaves + wave) * 16u;
+  const uint32_t* lrow = p.logits + (size_t)row * p.logits_ld;
+  v4u x[4];
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    // past the last tile the row's last tile is read again (and not stored)
+    const uint32_t t = min(first + 4u * k + (lane >> 4), kTilesPerRow - 1u);
+    x[k] = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(lrow + t * kTileIds + 4u * n));
+  }
+  float* buf = turn[wave];
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k)
+    *reinterpret_cast<v4u*>(buf + (4u * k + (lane >> 4)) * kTailStride + 4u * n) = x[k];
+  __builtin_amdgcn_wave_barrier();
+  const uint32_t qd = lane & 3u;
+  uint32_t word, second;
+  four_lane_words(buf + (lane >> 2) * kTailStride + 16u * qd, qd, word, second);
+  const uint32_t tile = first + (lane >> 2);
+  if (qd == 0u && tile < kTilesPerRow) {
+    p.tilemax[(size_t)row * kTilesPerRow + tile] = word;
+    p.tilesec[(size_t)row * kTilesPerRow + tile] = second;
   }
 }
 
@@ -2390,26 +2449,17 @@ hipError_t launch_lm_sample(const LmParams& p, const RowParams& rp, hipStream_t 
 
 hipError_t launch_tile_select(const LmParams& p, const RowParams& rp, hipStream_t stream) {
   (void)hipGetLastError();  // report only this call's launch errors
-  // Logits in HBM: two loads per thread, 75 workgroups per row (B = 1, 16,
-  // 64, 192 steps 0.6, 0.6, 0.4, 0.2 us shorter than with four; one load or
-  // eight were slower from 16 rows up).  Up to three rows, where 75
-  // workgroups per row leave CUs idle, one load, 149 workgroups per row:
-  // B = 1, 2, 3 cold steps 7.8, 8.2, 8.3 -> 7.6, 7.9, 8.1 us (wall, one box;
-  // 64 or 128 threads per workgroup measured the same).  Logits in pinned
-  // host memory: four, 38 workgroups.
-  if (p.logits_copy == nullptr && p.rows <= 3u) {
-    constexpr uint32_t kGroupTiles = 16u;
-    hipLaunchKernelGGL(tile_words_kernel<1>,
-                       dim3((kTilesPerRow + kGroupTiles - 1) / kGroupTiles, p.rows), dim3(256), 0,
-                       stream, p);
-  } else if (p.logits_copy == nullptr) {
-    constexpr uint32_t kGroupTiles = 16u * 2u;
-    hipLaunchKernelGGL(tile_words_kernel<2>,
-                       dim3((kTilesPerRow + kGroupTiles - 1) / kGroupTiles, p.rows), dim3(256), 0,
-                       stream, p);
+  if (p.logits_copy == nullptr) {
+    // up to three rows leave CUs idle: one wave per workgroup, 149 a row
+    const uint32_t waves = p.rows <= 3u ? 1u : 2u;
+    const dim3 grid((kTilesPerRow + 16u * waves - 1) / (16u * waves), p.rows);
+    if (waves == 1u)
+      hipLaunchKernelGGL(tile_words_kernel<1>, grid, dim3(64), 0, stream, p);
+    else
+      hipLaunchKernelGGL(tile_words_kernel<2>, grid, dim3(128), 0, stream, p);
   } else {
     constexpr uint32_t kGroupTiles = 16u * 4u;
-    hipLaunchKernelGGL(tile_words_kernel<4>,
+    hipLaunchKernelGGL(tile_words_copy_kernel,
                        dim3((kTilesPerRow + kGroupTiles - 1) / kGroupTiles, p.rows), dim3(256), 0,
                        stream, p);
   }
