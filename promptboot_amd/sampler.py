@@ -579,7 +579,7 @@ class DecodeBatch:
     def active(self) -> bool:
         return bool((self.row_state_host == ROW_ACTIVE).any())
 
-    def _draw(self, stream):
+    def _draw(self, stream=None):
         """One uniform per active row, on its way to the device on `stream`."""
         before = self.row_state_host.copy()
         # whatever produces the step's input has run, and no copy of an earlier
@@ -594,7 +594,7 @@ class DecodeBatch:
         for r in range(self.rows):
             self.states[r] = self._saved[r]
 
-    def _settle(self, before, stream):
+    def _settle(self, before, stream=None):
         out = 4 * self.rows
         hip.copy_async(self._host.data_ptr() + out, self._io.data_ptr() + out, 2 * out, hip.D2H,
                        stream)
