@@ -786,11 +786,11 @@ def measured_traffic(version: str) -> dict:
 LM_STEP_KERNELS = {
     ("q4_0", 256): [("pb::lm_quant_kernel", 57344),
                     ("pb::lm_gemm_kernel<false, false, 28u>", 1215488),
-                    ("pb::lm_select_kernel<1>", 131072)],
+                    ("pb::lm_select_kernel<1, false>", 131072)],
     ("q8_0", 256): [("pb::lm_quant_kernel", 57344), ("pb::lm_gemm_kernel<true, false, 0u>", 1215488),
-                    ("pb::lm_select_kernel<2>", 131072)],
-    ("q4_0", 1): [("pb::lm_gemm_narrow_kernel<false", 152064), ("pb::lm_select_kernel<0>", 512)],
-    ("q8_0", 1): [("pb::lm_gemm_narrow_kernel<true", 151936), ("pb::lm_select_kernel<0>", 512)],
+                    ("pb::lm_select_kernel<2, false>", 131072)],
+    ("q4_0", 1): [("pb::lm_gemm_narrow_kernel<false", 152064), ("pb::lm_select_kernel<0, false>", 512)],
+    ("q8_0", 1): [("pb::lm_gemm_narrow_kernel<true", 151936), ("pb::lm_select_kernel<0, false>", 512)],
 }
 
 

@@ -73,10 +73,10 @@ constexpr uint32_t kGemmThreads = 256;  // four waves
 // (same box, traced).  16 or 64 rows per wave were slower (+9 % and +2.5 %:
 // the nibble unpacking is shared by a wave's rows; 64 rows need 213 VGPRs).
 constexpr uint32_t kRowsPerGroup = 128;
-// Batches up to kNarrowRows take lm_gemm_narrow_kernel (measured per step,
-// Q4_0 / Q8_0: B = 64 43.2 / 54.6 us against 57 / 69 for 65 rows with the wide
-// kernel; B = 100 68.5 / 85.6 with four row groups of the narrow form, against
-// 64.1 / 81.5 wide).
+// Batches up to kNarrowRows take lm_gemm_narrow_kernel.  Measured per step on
+// one box, Q4_0 / Q8_0: 64 rows 46.2 / 56.8 us, 65 rows with the wide kernel
+// 53.3 / 68.5; 100 rows 68.5 / 85.6 with four row groups of the narrow form,
+// 64.1 / 81.5 wide.
 constexpr uint32_t kWordsPerRow = kVocab / 32;
 // Blocks of 32 in Qwen2.5-0.5B's hidden state of 896: the width whose block
 // loops are unrolled whole.
