@@ -969,7 +969,8 @@ __device__ __forceinline__ void write_tile(const LmParams& p, const v4f (&total)
   const float* mine = buf + (lane >> 2) * kTailStride + 16u * qd;
   auto pass = [&](auto half_tag) __attribute__((always_inline)) {
     constexpr int half = decltype(half_tag)::value;
-    // the rows past kRegs are left as they are: their words are not stored
+    // the rows past kRegs are left as they are: their words are not stored (they are the next
+    // group's rows when a group has fewer than 32)
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       const int i = 8 * half + r;
@@ -980,7 +981,7 @@ __device__ __forceinline__ void write_tile(const LmParams& p, const v4f (&total)
     __builtin_amdgcn_wave_barrier();
     uint32_t word, second;
     four_lane_words(mine, qd, word, second);
-    if (qd == 0u) {
+    if (qd == 0u && 16u * (uint32_t)half + (lane >> 2) < 2u * (uint32_t)kRegs) {
       const uint32_t off = ((wave_row + 16u * (uint32_t)half + (lane >> 2)) * kTilesPerRow + tile) * 4u;
       __builtin_amdgcn_raw_buffer_store_b32(word, tm, off, 0, 0);
       __builtin_amdgcn_raw_buffer_store_b32(second, ts, off, 0, 0);
@@ -994,7 +995,7 @@ __device__ __forceinline__ void write_tile(const LmParams& p, const v4f (&total)
 // ---- the head for narrow batches (up to 64 rows) ----
 // The wide kernel stages the scales of 128 rows in LDS and gives the four
 // waves of a workgroup one 64-id tile; with few rows most of that work is
-// padding.  Here a wave takes one tile and one group of 32 rows (kGroups row
+// padding.  Here a wave takes one tile and one group of up to 32 rows (kGroups row
 // groups per workgroup, so that a tile's weights are read by the waves of one
 // workgroup), and of its 16 result registers per column tile only the kRegs
 // that hold real rows go through the epilogue: registers 0 .. 3 of both lane
@@ -1038,9 +1039,13 @@ __device__ __forceinline__ void write_tile(const LmParams& p, const v4f (&total)
 // four row groups and LDS-staged weight scales was no faster than the wide
 // kernel: 256 rows 116-125 us a step against 115-122.)
 constexpr uint32_t kMaxBlocks = 2048 / 32;
+// A row group's rows: 32, or with several groups those that kRegs result
+// registers of both lane halves hold.
+constexpr uint32_t narrow_group_rows(int groups, int regs) { return groups > 1 ? 2u * (uint32_t)regs : 32u; }
 template <bool kQ8, int kGroups, int kRegs, bool kFused, int kWaves>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRegs >= 12 && !(kQ8 && kGroups == 1) ? 3 : 4))) void lm_gemm_narrow_kernel(LmParams p) {
-  constexpr uint32_t kRows = 32u * kGroups;      // rows per workgroup
+  constexpr uint32_t kGroupRows = narrow_group_rows(kGroups, kRegs);
+  constexpr uint32_t kRows = kGroupRows * kGroups;  // rows per workgroup
   constexpr uint32_t kTiles = kWaves / kGroups;  // tiles per workgroup
   constexpr uint32_t kThreads = 64u * kWaves;
   constexpr int kQuads = (kRegs + 3) / 4;        // result quads in use
@@ -1072,7 +1077,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRe
   const uint32_t tile_raw = item / gridDim.y * kTiles + wave / kGroups;
   const uint32_t tile = min(tile_raw, kTilesPerRow - 1u);
   const uint32_t group0 = item % gridDim.y * kRows;
-  const uint32_t wave_row = wave % kGroups * 32u;  // first row inside the workgroup's rows
+  const uint32_t wave_row = wave % kGroups * kGroupRows;  // first row inside the workgroup's rows
   const uint32_t rw0 = group0 + wave_row;
   const bool live = rw0 < p.rows && tile_raw < kTilesPerRow;  // else the whole wave idles
   constexpr uint32_t kTile = kQ8 ? kTileBytesQ8 : kTileBytes;
@@ -1185,7 +1190,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRe
         const uint32_t r = 4u * (t % kRowQuads);
         if (t < quads)
           *reinterpret_cast<v4u*>(
-              &act_scale[(r >> 5) * group_words + t / kRowQuads * 32u + (r & 31u)]) = as[k];
+              &act_scale[r / kGroupRows * group_words + t / kRowQuads * 32u + r % kGroupRows]) = as[k];
       }
     }
   }
@@ -2387,7 +2392,7 @@ static void launch_gemm_wide(const LmParams& p, hipStream_t stream) {
 template <bool kQ8, int kGroups, int kRegs, bool kFused, int kWaves>
 static void launch_gemm(const LmParams& p, hipStream_t stream) {
   constexpr uint32_t kTiles = kWaves / kGroups;
-  constexpr uint32_t kRows = 32u * kGroups;
+  constexpr uint32_t kRows = narrow_group_rows(kGroups, kRegs) * kGroups;
   const uint32_t blocks = p.cols / 32u;
   const dim3 grid((kTilesPerRow + kTiles - 1) / kTiles, (p.rows + kRows - 1) / kRows);
   uint32_t words = kGroups * blocks * 32u + (uint32_t)kWaves * kTailWords;
@@ -2398,16 +2403,20 @@ static void launch_gemm(const LmParams& p, hipStream_t stream) {
 }
 
 // Result registers by rows (their epilogue is the work that grows with them),
-// and from 33 rows two row groups per workgroup.  Workgroups of four waves, two
+// and from 33 rows two row groups per workgroup: of 24 rows up to 48 rows, of 32
+// above.  (33 to 48 rows as 32 and the rest left a quarter of the epilogue to
+// padding: 40 rows Q4_0 43.5 -> 40.1 us, Q8_0 52.0 -> 50.4; 48 rows 43.8 ->
+// 41.2 and 53.5 -> 51.9; two-wave workgroups and, for the Q8_0 head, four waves
+// per SIMD were no faster.)  Workgroups of four waves, two
 // for the Q8_0 head with one row group (one row 35.0 -> 33.2 us, 16 rows 42.0
 // -> 38.8: 594 workgroups of four leave some CUs three and others two).
 // Measured per step (us) against one or two row tiles of 16 rows on
 // v_mfma_i32_16x16x32_i8 with the scales loaded beside the operands:
 //   rows      1     4     8     16    24    32    40    64
 //   Q4_0      20.1  26.2  27.3  27.8  38.0  38.3  55.8  56.9
-//     now     20.5  21.9  22.7  25.4  28.0  31.4  41.5  43.2
+//     now     20.5  21.9  22.7  25.4  28.0  31.4  40.1  43.2
 //   Q8_0      33.1  35.8  37.5  38.7  57.9  58.8  66.8  70.6
-//     now     31.4  34.7  35.4  37.5  40.1  42.4  51.3  54.6
+//     now     31.4  34.7  35.4  37.5  40.1  42.4  50.4  54.6
 template <bool kQ8>
 static void launch_gemm_rows(const LmParams& p, hipStream_t stream) {
   if (p.rows > kNarrowRows) return launch_gemm_wide<kQ8>(p, stream);
@@ -2419,6 +2428,7 @@ static void launch_gemm_rows(const LmParams& p, hipStream_t stream) {
   if (p.rows <= 16) return launch_gemm<kQ8, 1, 8, false, kW>(p, stream);
   if (p.rows <= 24) return launch_gemm<kQ8, 1, 12, false, kW>(p, stream);
   if (p.rows <= 32) return launch_gemm<kQ8, 1, 16, false, kW>(p, stream);
+  if (p.rows <= 48) return launch_gemm<kQ8, 2, 12, false, 4>(p, stream);
   return launch_gemm<kQ8, 2, 16, false, 4>(p, stream);
 }
 

@@ -111,3 +111,31 @@ def test_narrow_head_either_side_of_every_row_count_it_branches_on(smp, q8, cols
         rtok, _, _, _ = o.sample_batch(rlog[:rows], np.zeros((rows, 1), np.uint32),
                                        np.zeros(rows, np.uint32), r24, threads=4)
         assert (token.cpu().numpy().view(np.uint32) == rtok).all(), (cols, rows)
+
+
+@pytest.mark.parametrize("q8", [False, True], ids=["q4_0", "q8_0"])
+@pytest.mark.parametrize("rows", [33, 40, 47, 48, 49])
+def test_two_row_groups_of_24_rows(smp, q8, rows):
+    """33 to 48 rows take two groups of 24 rows, 49 two of 32: logits and draws
+    of every row, the first group's last rows and the second's first among
+    them, at an odd number of blocks.  Defined bit for bit, so they must agree."""
+    import torch
+
+    cols = 160
+    head = make_head(cols, q8, seed=rows + (2000 if q8 else 0))
+    packed = smp.pack_lmhead(torch.from_numpy(head).to("cuda:0"), q8=q8, cols=cols)
+    hidden = np.random.default_rng(rows).standard_normal((rows, cols)).astype(np.float32)
+    rlog = o.lmhead_logits(hidden, head, V, cols, threads=16, q8=q8)
+    rnan = np.isnan(rlog.view(np.float32))
+    r24 = (np.arange(rows, dtype=np.uint32) * 104729 + 11) & 0xFFFFFF
+    token = torch.empty(rows, dtype=torch.int32, device="cuda:0")
+    logits = torch.full((rows + 1, V), -1, dtype=torch.int32, device="cuda:0")
+    smp.lmhead_sample(packed, to_dev(hidden), to_dev(r24), token=token, logits=logits, cols=cols, q8=q8)
+    torch.cuda.synchronize()
+    glog = logits.cpu().numpy().view(np.uint32)
+    assert (glog[rows] == 0xFFFFFFFF).all()  # nothing past the last row
+    assert (np.isnan(glog[:rows].view(np.float32)) == rnan).all()
+    assert ((glog[:rows] == rlog) | rnan).all()
+    rtok, _, _, _ = o.sample_batch(rlog, np.zeros((rows, 1), np.uint32), np.zeros(rows, np.uint32), r24,
+                                   threads=4)
+    assert (token.cpu().numpy().view(np.uint32) == rtok).all()
