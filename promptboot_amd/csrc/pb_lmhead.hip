@@ -896,12 +896,13 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
 // ones).
 //
 // Every store goes through a resource over the group's real rows: a padding
-// row's store falls outside it and is dropped, so no store needs a row test,
-// and each address is the lane's 32-bit offset plus the step's.  The logits
+// row's store falls outside it and is dropped, so no store needs a row test.
+// The row is in the vector offset whole: the range check covers that offset,
+// and says nothing about a scalar one that reaches past the resource by
+// itself (9, 10, 17, 18, 25 and 26 rows have such padding rows).  The logits
 // are non-temporal: the selection reads a few tiles of them, and ordinary
-// stores of a 256-row step (155.6 MB) evict the packed weights that a
-// workgroup's waves share through the L2 (Q8_0 step of 256 rows: 161.3-162.0
-// -> 142.1-149.8 us).
+// stores would evict the packed weights that a workgroup's waves share
+// through the L2.
 //
 // The words go through LDS (buf: the wave's own 16 rows of kTailStride
 // words), sixteen rows at a time, so that four lanes hold a row, sixteen ids
@@ -930,8 +931,8 @@ __device__ __forceinline__ void write_tile(const LmParams& p, const v4f (&total)
 #pragma unroll
   for (int i = 0; i < kRegs; ++i)
     __builtin_amdgcn_raw_buffer_store_b64(
-        v2u{b_of(total[0][i / 4][i % 4]), b_of(total[1][i / 4][i % 4])}, logits, off0,
-        (8u * ((uint32_t)i >> 2) + ((uint32_t)i & 3u)) * ld * 4u, kNonTemporal);
+        v2u{b_of(total[0][i / 4][i % 4]), b_of(total[1][i / 4][i % 4])}, logits,
+        off0 + (8u * ((uint32_t)i >> 2) + ((uint32_t)i & 3u)) * ld * 4u, 0, kNonTemporal);
   const __amdgpu_buffer_rsrc_t tm = __builtin_amdgcn_make_buffer_rsrc(
       p.tilemax + (size_t)base_row * kTilesPerRow, (short)0, (int)(real * kTilesPerRow * 4u),
       kBufferFlags);

@@ -139,3 +139,26 @@ def test_two_row_groups_of_24_rows(smp, q8, rows):
     rtok, _, _, _ = o.sample_batch(rlog, np.zeros((rows, 1), np.uint32), np.zeros(rows, np.uint32), r24,
                                    threads=4)
     assert (token.cpu().numpy().view(np.uint32) == rtok).all()
+
+
+@pytest.mark.parametrize("q8", [False, True], ids=["q4_0", "q8_0"])
+@pytest.mark.parametrize("rows", [3, 9, 10, 11, 17, 18, 19, 25, 26, 27, 33, 41, 49, 63])
+def test_padding_rows_store_nothing(smp, q8, rows):
+    """A row group's padding rows are computed with the real ones and must
+    leave the 32 rows after the last real one alone.  At 9, 10, 17, 18, 25 and
+    26 rows some result registers hold rows of which the first lies past the
+    whole batch."""
+    import torch
+
+    cols = 64
+    head = make_head(cols, q8, seed=rows + (2000 if q8 else 0))
+    packed = smp.pack_lmhead(torch.from_numpy(head).to("cuda:0"), q8=q8, cols=cols)
+    hidden = np.random.default_rng(rows + 50).standard_normal((rows, cols)).astype(np.float32)
+    r24 = (np.arange(rows, dtype=np.uint32) * 7919 + 3) & 0xFFFFFF
+    token = torch.empty(rows, dtype=torch.int32, device="cuda:0")
+    logits = torch.full((rows + 32, V), -1, dtype=torch.int32, device="cuda:0")
+    smp.lmhead_sample(packed, to_dev(hidden), to_dev(r24), token=token, logits=logits[:rows], cols=cols, q8=q8)
+    torch.cuda.synchronize()
+    got = logits.cpu().numpy().view(np.uint32)
+    assert (got[rows:] == 0xFFFFFFFF).all()
+    assert (got[:rows] == o.lmhead_logits(hidden, head, V, cols, threads=16, q8=q8)).all()
