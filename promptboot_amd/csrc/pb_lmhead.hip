@@ -20,8 +20,8 @@
 //                      logit; without one (kLogits false: one pass) it writes
 //                      no logits, only that word and the tile's second word (a
 //                      bound on its other logits and the maximum's index).
-//   lm_gemm_narrow_kernel  the same for up to 64 rows, one wave per tile and 32
-//                      rows on v_mfma_i32_32x32x32_i8,
+//   lm_gemm_narrow_kernel  the same for up to 64 rows, one wave per tile and up
+//                      to 32 rows on v_mfma_i32_32x32x32_i8,
 //                      logits always written (to the workspace if the caller
 //                      keeps none) with both words; with up to
 //                      kFusedQuantRows rows each workgroup quantises the
@@ -74,9 +74,9 @@ constexpr uint32_t kGemmThreads = 256;  // four waves
 // the nibble unpacking is shared by a wave's rows; 64 rows need 213 VGPRs).
 constexpr uint32_t kRowsPerGroup = 128;
 // Batches up to kNarrowRows take lm_gemm_narrow_kernel.  Measured per step on
-// one box, Q4_0 / Q8_0: 64 rows 46.2 / 56.8 us, 65 rows with the wide kernel
-// 53.3 / 68.5; 100 rows 68.5 / 85.6 with four row groups of the narrow form,
-// 64.1 / 81.5 wide.
+// one box (the same inputs each step), Q4_0 / Q8_0: 64 rows 40.9 / 44.5 us, 65
+// rows with the wide kernel 51.9 / 57.2.  With inputs taken in turn, 100 rows
+// were 68.5 / 85.6 in four row groups of the narrow form, 64.1 / 81.5 wide.
 constexpr uint32_t kWordsPerRow = kVocab / 32;
 // Blocks of 32 in Qwen2.5-0.5B's hidden state of 896: the width whose block
 // loops are unrolled whole.
@@ -882,11 +882,16 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
     write_tile_words<2, 4>(p, total, group0, kRowsPerGroup, lrow0 + 4u * q, tile, n);
 }
 
+// A value every lane holds alike, moved to a scalar register so that the
+// compiler branches and selects on it as a wave-uniform value.
+__device__ __forceinline__ uint32_t uniform(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+}
+
 // ---- a narrow wave's results for one 64-id tile ----
-// total[ct][i] of lane l = 32 h + j is row base_row + wave_row + 8 (i / 4) + 4 h + i % 4,
+// total[ct][i] of lane l = 32 h + j is row wave_row + 8 (i / 4) + 4 h + i % 4,
 // id 64 tile + 2 j + ct, for i < kRegs (the MFMA's result layout).
-// base_row is the first row of the workgroup's group of group_rows rows and
-// wave_row the wave's first row in it.
+// wave_row is the wave's first row.
 //
 // Stored for the real rows: the raw logits, and per (row, tile)
 // the order word of the largest raw logit (kNonFiniteTile when one of them is
@@ -895,7 +900,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
 // reads (it never raises a value, so the raw maximum bounds the penalised
 // ones).
 //
-// Every store goes through a resource over the group's real rows: a padding
+// Every store goes through a resource over the real rows: a padding
 // row's store falls outside it and is dropped, so no store needs a row test.
 // The row is in the vector offset whole: the range check covers that offset,
 // and says nothing about a scalar one that reaches past the resource by
@@ -916,17 +921,15 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
 // whose word is the order word of zero.
 template <int kRegs>
 __device__ __forceinline__ void write_tile(const LmParams& p, const v4f (&total)[2][(kRegs + 3) / 4],
-                                           uint32_t base_row, uint32_t group_rows,
                                            uint32_t wave_row, uint32_t tile, uint32_t lane,
                                            float* buf) {
   const uint32_t j = lane & 31u;
   const uint32_t h = lane >> 5;
-  const uint32_t real = p.rows > base_row ? min(p.rows - base_row, group_rows) : 0u;
-  // the LM heads' logits are [rows][PB_VOCAB]: a group's rows span at most
+  // the LM heads' logits are [rows][PB_VOCAB]: the rows span at most
   // 64 x 151,936 words
   const uint32_t ld = (uint32_t)p.logits_ld;
   const __amdgpu_buffer_rsrc_t logits = __builtin_amdgcn_make_buffer_rsrc(
-      p.logits + (size_t)base_row * ld, (short)0, (int)(real * ld * 4u), kBufferFlags);
+      p.logits, (short)0, (int)(p.rows * ld * 4u), kBufferFlags);
   const uint32_t off0 = ((wave_row + 4u * h) * ld + tile * kTileIds + 2u * j) * 4u;
 #pragma unroll
   for (int i = 0; i < kRegs; ++i)
@@ -934,11 +937,9 @@ __device__ __forceinline__ void write_tile(const LmParams& p, const v4f (&total)
         v2u{b_of(total[0][i / 4][i % 4]), b_of(total[1][i / 4][i % 4])}, logits,
         off0 + (8u * ((uint32_t)i >> 2) + ((uint32_t)i & 3u)) * ld * 4u, 0, kNonTemporal);
   const __amdgpu_buffer_rsrc_t tm = __builtin_amdgcn_make_buffer_rsrc(
-      p.tilemax + (size_t)base_row * kTilesPerRow, (short)0, (int)(real * kTilesPerRow * 4u),
-      kBufferFlags);
+      p.tilemax, (short)0, (int)(p.rows * kTilesPerRow * 4u), kBufferFlags);
   const __amdgpu_buffer_rsrc_t ts = __builtin_amdgcn_make_buffer_rsrc(
-      p.tilesec + (size_t)base_row * kTilesPerRow, (short)0, (int)(real * kTilesPerRow * 4u),
-      kBufferFlags);
+      p.tilesec, (short)0, (int)(p.rows * kTilesPerRow * 4u), kBufferFlags);
   if constexpr (kRegs <= 2) {
     // One or two rows, in the registers of lanes 0 .. 31: reduced there, with
     // no round trips through LDS at the end of a step that is all latency
@@ -1043,6 +1044,8 @@ constexpr uint32_t kMaxBlocks = 2048 / 32;
 // A row group's rows: 32, or with several groups those that kRegs result
 // registers of both lane halves hold.
 constexpr uint32_t narrow_group_rows(int groups, int regs) { return groups > 1 ? 2u * (uint32_t)regs : 32u; }
+// Workgroups of `tiles` tiles each.
+constexpr uint32_t narrow_workgroups(uint32_t tiles) { return (kTilesPerRow + tiles - 1u) / tiles; }
 template <bool kQ8, int kGroups, int kRegs, bool kFused, int kWaves>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRegs >= 12 && !(kQ8 && kGroups == 1) ? 3 : 4))) void lm_gemm_narrow_kernel(LmParams p) {
   constexpr uint32_t kGroupRows = narrow_group_rows(kGroups, kRegs);
@@ -1051,7 +1054,13 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRe
   constexpr uint32_t kThreads = 64u * kWaves;
   constexpr int kQuads = (kRegs + 3) / 4;        // result quads in use
   constexpr uint32_t kSets = kQ8 && kGroups == 1 ? 1 : 2;
-  constexpr uint32_t kActSets = kSets;
+  // Q4_0: the weight scale's conversion, folded into the epilogue's fma, keeps
+  // the packed word alive past the load that replaces it, and the loop then
+  // ends with a wait for every load in flight to move that word into place.
+  // Converted ahead of it (us a step, folded / ahead): 1 row 20.0 / 19.8, 4
+  // 21.4 / 21.0, 24 28.7 / 27.1, 40 39.3 / 35.9, 64 43.2 / 41.2; but 5 rows
+  // 22.3 / 22.6, 8 22.5 / 23.1, 12 24.4 / 24.7, 16 24.6 / 24.3.
+  constexpr bool kConvertEarly = !kQ8 && (kFused || kRegs >= 12);
   static_assert(!kFused || (kGroups == 1 && kRegs <= 4), "fused rows fit one result quad");
   // Dynamic LDS: the activation scales (/ 16 for Q4_0) by row group, block and row; kFused: then
   // each block's quants, a real row's eight words each and a row of zeros.
@@ -1065,22 +1074,15 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRe
   const uint32_t j = lane & 31u;  // MFMA row (A) / column (B)
   const uint32_t h = lane >> 5;   // contraction half; result rows 8 g + 4 h + ..
   // Consecutive tiles run on the same XCD (xcd_contiguous_item): every
-  // (row, tile) gets two 4-byte words in row-major arrays, and the
-  // words of up to eight neighbouring tiles share a 32-byte sector, which
-  // leaves an XCD's L2 whole only when the neighbours were written through
-  // that L2.  With tile = block index the neighbours sat on eight different
-  // XCDs: 8 x the words' bytes written (39.7 MB instead of 4.9 MB per
-  // 256-row one-pass step, WRITE_SIZE).  The row groups of one tile are
-  // consecutive items, so they run on one XCD at about the same time and the
-  // head leaves HBM once (group-major items read it once per group).
-  const uint32_t item = xcd_contiguous_item(blockIdx.x + blockIdx.y * gridDim.x,
-                                            gridDim.x * gridDim.y);
-  const uint32_t tile_raw = item / gridDim.y * kTiles + wave / kGroups;
+  // (row, tile) gets two 4-byte words in row-major arrays, and the words of up
+  // to eight neighbouring tiles share a 32-byte sector, which leaves an XCD's
+  // L2 whole only when the neighbours were written through that L2.  A
+  // workgroup takes every row of its tiles, so the grid is a constant.
+  const uint32_t tile_raw =
+      xcd_contiguous_item(blockIdx.x, narrow_workgroups(kTiles)) * kTiles + wave / kGroups;
   const uint32_t tile = min(tile_raw, kTilesPerRow - 1u);
-  const uint32_t group0 = item % gridDim.y * kRows;
-  const uint32_t wave_row = wave % kGroups * kGroupRows;  // first row inside the workgroup's rows
-  const uint32_t rw0 = group0 + wave_row;
-  const bool live = rw0 < p.rows && tile_raw < kTilesPerRow;  // else the whole wave idles
+  const uint32_t wave_row = wave % kGroups * kGroupRows;  // the wave's first row
+  const bool live = wave_row < p.rows && tile_raw < kTilesPerRow;  // else the whole wave idles
   constexpr uint32_t kTile = kQ8 ? kTileBytesQ8 : kTileBytes;
   // The operands are buffer loads: a lane's byte offset is fixed, the block's
   // offset is a scalar, so a load costs no VALU address arithmetic (three to
@@ -1092,12 +1094,12 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRe
   const uint32_t w_off = tile * kTile + (kQ8 ? 1024u * h + 16u * j : 512u * h + 8u * j);
   const uint32_t s_off = tile * (2u * kTileIds) + 4u * j;
   const uint32_t a_stride = p.rows_pad * 32u;  // bytes per block
-  const uint32_t a_off = (rw0 + j) * 32u + 16u * h;
+  const uint32_t a_off = (wave_row + j) * 32u + 16u * h;
   const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint8_t*>(p.weights), (short)0, (int)(blocks * w_stride), kBufferFlags);
   const __amdgpu_buffer_rsrc_t ws_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint8_t*>(p.weights) + (size_t)blocks * w_stride, (short)0,
-      (int)(blocks * kVocab * 2u), kBufferFlags);
+      (int)(blocks * kVocab * 2u + (kQ8 ? 0u : kTilesPerRow * 4u)), kBufferFlags);
   const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<int8_t*>(p.act_q), (short)0, kFused ? 0 : (int)(blocks * a_stride), kBufferFlags);
   float* tail_lds = lds + kGroups * group_words;  // a buffer per wave
@@ -1124,26 +1126,30 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRe
     }
     o.ws = __builtin_amdgcn_raw_buffer_load_b32(ws_rsrc, s_off, b * (kVocab * 2u), 0);
   };
-  v4i act[kActSets];
+  v4i act[kSets];
   auto load_a = [&](uint32_t b, v4i& a) __attribute__((always_inline)) {
     if constexpr (kFused)
       a = *reinterpret_cast<const v4i*>(&aq_lds[b * aq_stride + aq_off]);
     else
       a = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_off, b * a_stride, 0));
   };
-  // a Q4_0 tile with an infinite or NaN weight scale (flagged at pack time)
-  const bool odd_tile =
-      !kQ8 && row_word(reinterpret_cast<const uint32_t*>(p.weights + (size_t)blocks * kVocab * 18) + tile) != 0u;
   // The first blocks' weights are requested before the scales are staged (or
   // the rows quantised), so their latency overlaps that and its barrier.
   Operands ops[kSets];
   const uint32_t last = blocks - 1u;
+  // The word that flags a Q4_0 tile with an infinite or NaN weight scale (set
+  // at pack time, after the scales) comes with them, as a vector load: a scalar
+  // one was waited for with the next kernel argument, a round trip to HBM
+  // before the rows' quantisation could start (one row 20.35 -> 20.15 us).
+  uint32_t odd_word = 0;
   if (live) {
 #pragma unroll
     for (uint32_t k = 0; k < kSets; ++k) load_w(min(k, last), ops[k]);
+    if constexpr (!kQ8)
+      odd_word = __builtin_amdgcn_raw_buffer_load_b32(ws_rsrc, blocks * (kVocab * 2u) + 4u * tile, 0, 0);
     if constexpr (!kFused) {
 #pragma unroll
-      for (uint32_t k = 0; k < kActSets; ++k) load_a(min(k, last), act[k]);
+      for (uint32_t k = 0; k < kSets; ++k) load_a(min(k, last), act[k]);
     }
   }
 
@@ -1166,11 +1172,12 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRe
           v4u{0u, 0u, 0u, 0u};
   } else {
     // Staged four rows per thread and load (16 bytes; rows_pad is a multiple
-    // of 64, so four rows are all inside the padded batch or all past it), four
-    // loads requested before any is stored.  Rows past the padded batch (only
-    // idle waves use them) read at the end of the resource, which returns
-    // zeros.  lm_quant_kernel stores a_scale / 16 for the Q4_0 epilogue and
-    // a_scale for the Q8_0 one.
+    // of 64, so every row staged is in the padded batch), four loads requested
+    // before any is stored; past the last block they return zeros.  The test of
+    // the row never fails: without it the compiler moves each load under its
+    // store's test (Q8_0, 8 to 48 rows: 0.2-0.3 us more a step).
+    // lm_quant_kernel stores a_scale / 16 for the Q4_0 epilogue and a_scale for
+    // the Q8_0 one.
     const uint32_t as_bytes = blocks * p.rows_pad * 4u;
     const __amdgpu_buffer_rsrc_t s_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         p.act_s, (short)0, (int)as_bytes, kBufferFlags);
@@ -1181,7 +1188,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRe
 #pragma unroll
       for (uint32_t k = 0; k < 4; ++k) {
         const uint32_t t = t0 + k * kThreads;
-        const uint32_t r = group0 + 4u * (t % kRowQuads);
+        const uint32_t r = 4u * (t % kRowQuads);
         const uint32_t off = r < p.rows_pad ? ((t / kRowQuads) * p.rows_pad + r) * 4u : as_bytes;
         as[k] = __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, off, 0, 0);
       }
@@ -1199,7 +1206,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRe
   if (!live) return;  // whole wave idle (no barrier follows)
   if constexpr (kFused) {
 #pragma unroll
-    for (uint32_t k = 0; k < kActSets; ++k) load_a(min(k, last), act[k]);
+    for (uint32_t k = 0; k < kSets; ++k) load_a(min(k, last), act[k]);
   }
 
   v16i magic;
@@ -1233,6 +1240,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRe
   // the block's weight scale of column tile ct, in the epilogue's form
   auto scale = [&](const Operands& o, int ct) __attribute__((always_inline)) {
     ws[ct] = __half2float(__ushort_as_half((unsigned short)(o.ws >> (16 * ct))));
+    if constexpr (kConvertEarly) __asm__("" : "+v"(ws[ct]));  // not folded into the epilogue
     if constexpr (!kQ8) wn[ct] = ws[ct] * -kMagic;
   };
   auto epilogue = [&](int ct, int g) __attribute__((always_inline)) {
@@ -1250,14 +1258,14 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRe
     }
   };
   // Block b: its weights in o (column tile 0's operand in w) and activations
-  // in a, the next block's weights in o1; the operands kSets (kActSets) blocks ahead
-  // are requested into o and a.
+  // in a, the next block's weights in o1; the operands kSets blocks ahead are
+  // requested into o and a.
   auto block = [&](uint32_t b, Operands& o, Operands& o1, v4i& a, v4i& a1) __attribute__((always_inline)) {
     const uint32_t ahead = min(b + 1u, last);
     scale(o, 1);
     w = operand(o, 1);
     d[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, w, magic, 0, 0, 0);
-    load_a(min(b + kActSets, last), a);
+    load_a(min(b + kSets, last), a);
     load_w(min(b + kSets, last), o);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1285,15 +1293,15 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRe
   for (; b + kSets <= blocks; b += kSets) {
 #pragma unroll
     for (uint32_t k = 0; k < kSets; ++k)
-      block(b + k, ops[k], ops[(k + 1) % kSets], act[k % kActSets], act[(k + 1) % kActSets]);
+      block(b + k, ops[k], ops[(k + 1) % kSets], act[k % kSets], act[(k + 1) % kSets]);
   }
 #pragma unroll
   for (uint32_t k = 0; k + 1 < kSets; ++k)
     if (b + k < blocks)
-      block(b + k, ops[k], ops[(k + 1) % kSets], act[k % kActSets], act[(k + 1) % kActSets]);
+      block(b + k, ops[k], ops[(k + 1) % kSets], act[k % kSets], act[(k + 1) % kSets]);
   if constexpr (!kQ8) {
     // Block by block again with the subtract-then-multiply form.
-    if (odd_tile) {
+    if (uniform(odd_word) != 0u) {
 #pragma unroll
       for (int ct = 0; ct < 2; ++ct) {
 #pragma unroll
@@ -1321,15 +1329,9 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(kRe
   // the lane number anew: nothing that the tail derives from it is kept through the loop
   uint32_t none = 0;
   __asm__ volatile("" : "+s"(none));
-  write_tile<kRegs>(p, total, group0, kRows, wave_row, tile,
+  write_tile<kRegs>(p, total, wave_row, tile,
                              __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, none)),
                              tail_lds + wave * kTailWords);
-}
-
-// A value every lane holds alike, moved to a scalar register so that the
-// compiler branches and selects on it as a wave-uniform value.
-__device__ __forceinline__ uint32_t uniform(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
 }
 
 // Collects into `cand` every key of this lane (keys[0..N)) in [lo, hi);
@@ -2393,9 +2395,8 @@ static void launch_gemm_wide(const LmParams& p, hipStream_t stream) {
 template <bool kQ8, int kGroups, int kRegs, bool kFused, int kWaves>
 static void launch_gemm(const LmParams& p, hipStream_t stream) {
   constexpr uint32_t kTiles = kWaves / kGroups;
-  constexpr uint32_t kRows = narrow_group_rows(kGroups, kRegs) * kGroups;
   const uint32_t blocks = p.cols / 32u;
-  const dim3 grid((kTilesPerRow + kTiles - 1) / kTiles, (p.rows + kRows - 1) / kRows);
+  const dim3 grid(narrow_workgroups(kTiles));  // every row is in a workgroup's groups
   uint32_t words = kGroups * blocks * 32u + (uint32_t)kWaves * kTailWords;
   if (kFused) words += blocks * (p.rows + 1u) * 8u;
   const size_t lds = words * sizeof(float);
@@ -2406,18 +2407,19 @@ static void launch_gemm(const LmParams& p, hipStream_t stream) {
 // Result registers by rows (their epilogue is the work that grows with them),
 // and from 33 rows two row groups per workgroup: of 24 rows up to 48 rows, of 32
 // above.  (33 to 48 rows as 32 and the rest left a quarter of the epilogue to
-// padding: 40 rows Q4_0 43.5 -> 40.1 us, Q8_0 52.0 -> 50.4; 48 rows 43.8 ->
-// 41.2 and 53.5 -> 51.9; two-wave workgroups and, for the Q8_0 head, four waves
-// per SIMD were no faster.)  Workgroups of four waves, two
-// for the Q8_0 head with one row group (one row 35.0 -> 33.2 us, 16 rows 42.0
-// -> 38.8: 594 workgroups of four leave some CUs three and others two).
-// Measured per step (us) against one or two row tiles of 16 rows on
-// v_mfma_i32_16x16x32_i8 with the scales loaded beside the operands:
+// padding: with inputs taken in turn, 40 rows Q4_0 43.5 -> 40.1 us, Q8_0 52.0
+// -> 50.4; 48 rows 43.8 -> 41.2 and 53.5 -> 51.9; two-wave workgroups and, for
+// the Q8_0 head, four waves per SIMD were no faster.)  Workgroups of four
+// waves, two for the Q8_0 head with one row group (one row 35.0 -> 33.2 us, 16
+// rows 42.0 -> 38.8: 594 workgroups of four leave some CUs three and others
+// two).  Measured per step (us, one box, the same inputs each step) against one
+// or two row tiles of 16 rows on v_mfma_i32_16x16x32_i8 with the scales loaded
+// beside the operands:
 //   rows      1     4     8     16    24    32    40    64
-//   Q4_0      20.1  26.2  27.3  27.8  38.0  38.3  55.8  56.9
-//     now     20.5  21.9  22.7  25.4  28.0  31.4  40.1  43.2
-//   Q8_0      33.1  35.8  37.5  38.7  57.9  58.8  66.8  70.6
-//     now     31.4  34.7  35.4  37.5  40.1  42.4  50.4  54.6
+//   Q4_0      19.7  25.8  26.9  27.6  38.2  38.8  56.2  57.3
+//     now     19.6  20.9  22.6  24.3  26.9  30.0  35.8  40.9
+//   Q8_0      28.6  32.3  32.7  33.5  55.4  56.1  58.4  60.1
+//     now     27.8  30.0  31.3  32.2  33.6  34.7  40.4  44.5
 template <bool kQ8>
 static void launch_gemm_rows(const LmParams& p, hipStream_t stream) {
   if (p.rows > kNarrowRows) return launch_gemm_wide<kQ8>(p, stream);
