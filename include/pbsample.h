@@ -442,10 +442,12 @@ uint32_t pb_device_penalize_bits(const uint32_t *d_in, uint32_t *d_out, size_t n
 /* One-wave self-test of the lane exchanges (DPP, permlane swaps) and wave
  * reductions the selection uses; writes 11 x 64 words to d_out. */
 uint32_t pb_device_wave_selftest(uint32_t *d_out, void *stream);
-/* One-wave self-test of the int8 MFMA fragment layout the LM head uses:
- * writes the 32 x 32 int32 product of A[i][k] = (7i + 3k) % 17 - 8 and
- * B[k][j] = (5k + 11j) % 15 - 7 (k < 32) to d_out[32 i + j]. */
+/* One-wave self-tests of the int8 MFMA fragment layouts the LM heads use, 16 x 16
+ * (above 64 rows) and 32 x 32 (up to 64): each writes the 32 x 32 int32 product of
+ * A[i][k] = (7i + 3k) % 17 - 8 and B[k][j] = (5k + 11j) % 15 - 7 (k < 32) to
+ * d_out[32 i + j]. */
 uint32_t pb_device_mfma_selftest(int32_t *d_out, void *stream);
+uint32_t pb_device_mfma32_selftest(int32_t *d_out, void *stream);
 
 /* Read-only stream probe (diagnostic, no reference counterpart): `blocks`
  * workgroups read the n_words words at d_in (16-byte aligned) with the

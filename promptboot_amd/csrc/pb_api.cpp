@@ -867,6 +867,12 @@ uint32_t pb_device_mfma_selftest(int32_t* d_out, void* stream) {
              : PB_DEVICE;
 }
 
+uint32_t pb_device_mfma32_selftest(int32_t* d_out, void* stream) {
+  return pb::launch_mfma32_selftest(d_out, static_cast<hipStream_t>(stream)) == hipSuccess
+             ? PB_OK
+             : PB_DEVICE;
+}
+
 }  // extern "C"
 
 // ---- single-row drop-ins on the default context ----

@@ -111,6 +111,7 @@ hipError_t launch_tile_select(const LmParams& p, const RowParams& rp, hipStream_
 constexpr uint32_t kTileSelectRows = PB_TILE_SELECT_ROWS;
 constexpr size_t kTileSelectBytesPerRow = (size_t)(PB_VOCAB / 64) * 8;
 hipError_t launch_mfma_selftest(int32_t* out, hipStream_t stream);
+hipError_t launch_mfma32_selftest(int32_t* out, hipStream_t stream);
 
 uint32_t segments_for_rows(uint32_t rows);
 // forced_segments == 0 picks segments_for_rows(rows).

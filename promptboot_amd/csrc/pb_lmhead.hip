@@ -2347,6 +2347,32 @@ __global__ __launch_bounds__(64) void mfma_selftest_kernel(int32_t* out) {
   }
 }
 
+// The same product as one 32 x 32 tile, with the narrow GEMM's contraction slots
+// and result registers.
+__global__ __launch_bounds__(64) void mfma32_selftest_kernel(int32_t* out) {
+  const uint32_t lane = lane_id();
+  const uint32_t j = lane & 31u;
+  const uint32_t h = lane >> 5;
+  v4i a, b;
+  for (uint32_t r = 0; r < 4; ++r) {
+    uint32_t aw = 0, bw = 0;
+    for (uint32_t c = 0; c < 4; ++c) {
+      const uint32_t k = 16u * (r & 1u) + 4u * (2u * h + (r >> 1)) + c;
+      const int av = (int)((7u * j + 3u * k) % 17u) - 8;
+      const int bv = (int)((5u * k + 11u * j) % 15u) - 7;
+      aw |= ((uint32_t)av & 0xffu) << (8 * c);
+      bw |= ((uint32_t)bv & 0xffu) << (8 * c);
+    }
+    a[r] = (int)aw;
+    b[r] = (int)bw;
+  }
+  v16i magic;
+  for (int i = 0; i < 16; ++i) magic[i] = (int)kMagicBits;
+  const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, magic, 0, 0, 0);
+  for (uint32_t i = 0; i < 16; ++i)
+    out[32u * (8u * (i >> 2) + 4u * h + (i & 3u)) + j] = (int32_t)(__int_as_float(d[i]) - kMagic);
+}
+
 hipError_t launch_lm_pack(const uint8_t* in, uint8_t* out, uint32_t vocab, uint32_t blocks,
                           hipStream_t stream) {
   (void)hipGetLastError();  // report only this call's launch errors
@@ -2495,6 +2521,12 @@ hipError_t launch_tile_select(const LmParams& p, const RowParams& rp, hipStream_
 hipError_t launch_mfma_selftest(int32_t* out, hipStream_t stream) {
   (void)hipGetLastError();  // report only this call's launch errors
   hipLaunchKernelGGL(mfma_selftest_kernel, dim3(1), dim3(64), 0, stream, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_mfma32_selftest(int32_t* out, hipStream_t stream) {
+  (void)hipGetLastError();  // report only this call's launch errors
+  hipLaunchKernelGGL(mfma32_selftest_kernel, dim3(1), dim3(64), 0, stream, out);
   return hipGetLastError();
 }
 

@@ -56,6 +56,22 @@ def test_mfma_fragment_layout():
     assert (out.cpu().numpy().reshape(32, 32) == want).all()
 
 
+def test_mfma_fragment_layout_of_the_narrow_head():
+    """One 32 x 32 x 32 tile: 16 contraction slots per half wave, result row
+    8 (i / 4) + 4 h + i % 4 in register i."""
+    import torch
+
+    out = torch.zeros(32 * 32, dtype=torch.int32, device="cuda:0")
+    st = s.lib().pb_device_mfma32_selftest(ctypes.c_void_p(out.data_ptr()),
+                                           ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert st == 0
+    torch.cuda.synchronize()
+    i = np.arange(32)[:, None]
+    k = np.arange(32)[None, :]
+    want = ((7 * i + 3 * k) % 17 - 8) @ ((5 * i + 11 * k) % 15 - 7)
+    assert (out.cpu().numpy().reshape(32, 32) == want).all()
+
+
 def run_head(smp, packed, hidden, hist, hist_len, r24, q8=False, cols=workloads.HIDDEN):
     import torch
 
@@ -79,7 +95,7 @@ def oracle_head(w, hidden, rows):
     return logits, tok, det, err
 
 
-# up to 64 rows the head runs lm_gemm_narrow_kernel (one 16-row tile per wave up
+# up to 64 rows the head runs lm_gemm_narrow_kernel (one group of rows per tile up
 # to 32 rows, two above), beyond that lm_gemm_kernel: both sides of each switch
 @pytest.mark.parametrize("rows", [1, 2, 5, 16, 17, 32, 33, 64, 65, 129, 300])
 def test_head_logits_and_draws_are_bit_exact(smp, head, rows):
