@@ -105,9 +105,14 @@ hipError_t launch_lm_sample(const LmParams& p, const RowParams& rp, hipStream_t 
 hipError_t launch_tile_select(const LmParams& p, const RowParams& rp, hipStream_t stream);
 // Batches up to this size take launch_tile_select (without a `seen`
 // scratch off 16-byte alignment or a forced slice plan): rows x 2,374 x 8 bytes of workspace.
-// Measured per step (us, tile selection / slice plan), full-context
-// histories: B = 128 34.3 / 36.1, 192 40.6 / 42.2, 255 47.5 / 45.7, 512
-// 87.7 / 63.2; histories of at most 4,096 ids, B = 128: 23.9 / 28.7.
+// Measured per step (us, tile selection / slice plan, the same inputs each
+// step), histories of up to 1,024 and up to 32,768 ids:
+//   rows        128          192          224          256          300          384
+//   1,024       18.6 / 25.9  26.8 / 31.5  28.9 / 33.1  33.7 / 33.6  40.9 / 42.3  50.4 / 44.6
+//   32,768      23.8 / 33.1  31.6 / 40.4  35.7 / 41.3  39.3 / 42.3  48.5 / 49.5  60.7 / 52.0
+// The two meet at 256 rows of short histories and past 300 of long ones.  The
+// line stays where the allocation-free entry point's workspace and the
+// header's PB_TILE_SELECT_ROWS have it.
 constexpr uint32_t kTileSelectRows = PB_TILE_SELECT_ROWS;
 constexpr size_t kTileSelectBytesPerRow = (size_t)(PB_VOCAB / 64) * 8;
 hipError_t launch_mfma_selftest(int32_t* out, hipStream_t stream);

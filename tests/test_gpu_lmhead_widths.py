@@ -1,8 +1,8 @@
 """Both LM heads at hidden widths other than the model's 896 (GPU).
 
 The GEMMs' block loops treat the first blocks and the last ones apart: the
-first block starts the running totals, loads run one (Q4_0) or two (Q8_0)
-blocks ahead, and an odd or short block count ends outside the loop.  The
+first block starts the running totals, loads run one or two blocks ahead
+by kernel and format, and an odd or short block count ends outside the loop.  The
 model's width (28 blocks) exercises none of the short or odd cases, so each
 head runs here at 1, 2, 3, 5 and 29 blocks, through the narrow kernel with
 its own quantisation (1 and 3 rows), the narrow kernel after lm_quant_kernel
